@@ -1002,11 +1002,11 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
-// One wave per (request, query head).  The partials of the first kSpecParts
-// pieces and the log2-sum-exps are loaded together with the request's piece
-// count (all inside the max_parts rows the workspace holds for the request),
-// so the common case costs one memory round trip; lane p weighs piece p and
-// every lane folds its D/64 dims.  Requests with a single piece were finished
+// One wave per (request, query head), for plans with at most kSpecParts pieces
+// per request.  The partials and the log2-sum-exps are loaded together with
+// the request's piece count (all inside the max_parts rows the workspace holds
+// for the request), so a merge costs one memory round trip; lane p weighs
+// piece p and every lane folds its D/64 dims.  Requests with a single piece were finished
 // by the streaming kernel; requests with no pages get a zero output and
 // lse = -inf.
 //
@@ -1032,7 +1032,7 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(MergeArgs a) {
   const int64_t lse0 = base * G + g;  // piece p at part_lse[lse0 + p * G]
   const int nparts_raw = a.req_nparts[b];
   const int nspec = have_parts ? min(max_parts, kSpecParts) : 0;
-  const float lse_spec = (have_parts && lane < min(max_parts, 64))
+  const float lse_spec = (have_parts && lane < max_parts)
                              ? a.part_lse[lse0 + int64_t(lane) * G] : -INFINITY;
   float po[kSpecParts][EPL];
 #pragma unroll
@@ -1043,11 +1043,9 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(MergeArgs a) {
   }
   const int nparts = min(nparts_raw, max_parts);
   if (nparts == 1) return;
-  const float* lp = have_parts ? a.part_lse + lse0 : nullptr;  // read only when nparts > 64
   uint16_t* out = a.out + int64_t(b) * a.out_stride + int64_t(hq) * D;
 
   float mx = lane < nparts ? lse_spec : -INFINITY;
-  for (int p = 64 + lane; p < nparts; p += 64) mx = fmaxf(mx, lp[int64_t(p) * G]);
   mx = wave_max(mx);
   if (nparts <= 0 || mx == -INFINITY) {
 #pragma unroll
@@ -1060,28 +1058,12 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(MergeArgs a) {
   for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
   const float w0 = lane < nparts ? fast_exp2(lse_spec - mx) : 0.f;
   float S = w0;
-  if (nparts <= kSpecParts) {
 #pragma unroll
-    for (int p = 0; p < kSpecParts; ++p) {
-      if (p < nparts) {
-        const float wp = readlane_f(w0, p);
+  for (int p = 0; p < kSpecParts; ++p) {
+    if (p < nparts) {
+      const float wp = readlane_f(w0, p);
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) acc[e] = fmaf(wp, po[p][e], acc[e]);
-      }
-    }
-  } else {
-    for (int q0 = 0; q0 < nparts; q0 += 64) {
-      const float w = q0 == 0 ? w0
-                              : (q0 + lane < nparts
-                                     ? fast_exp2(lp[int64_t(q0 + lane) * G] - mx) : 0.f);
-      if (q0 > 0) S += w;
-      const int cnt = min(64, nparts - q0);
-      for (int j = 0; j < cnt; ++j) {
-        const float wj = readlane_f(w, j);
-        const float* src = a.part_o + ((base + q0 + j) * G + g) * D + lane * EPL;
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) acc[e] = fmaf(wj, src[e], acc[e]);
-      }
+      for (int e = 0; e < EPL; ++e) acc[e] = fmaf(wp, po[p][e], acc[e]);
     }
   }
   S = wave_sum(S);
@@ -1089,6 +1071,93 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(MergeArgs a) {
 #pragma unroll
   for (int e = 0; e < EPL; ++e) out[lane * EPL + e] = f32_to_bf16(acc[e] * inv);
   if (a.lse && lane == 0) a.lse[int64_t(b) * Hq + hq] = (mx + fast_log2(S)) * kLn2;
+}
+
+// Plans whose requests may have more than kSpecParts pieces (few requests over
+// many segments): the same merge by four waves per (request, query head), wave
+// w folding pieces w, w + 4, ... with four partials in flight, the waves' sums
+// added through LDS.  Bound by latency: one wave alone folded them as a chain
+// of single loads, 15.7 us of a 28.1 us decode at 65 pieces (8 requests of
+// 300-2000 tokens, 8 KV heads; 18.3 us this way), and a decode of one request
+// of 4096 tokens (256 pieces) took 70.2 us against 25.2.  At 16 pieces and
+// fewer one wave's loads are already a single batch and its workgroup, with no
+// barrier, starts and ends sooner.
+constexpr int kManyWaves = 4;
+
+template <int D>
+__global__ __launch_bounds__(64 * kManyWaves) void decode_merge_many_kernel(MergeArgs a) {
+  constexpr int EPL = D / 64;     // dims per lane
+  constexpr int kAhead = 4;       // partials in flight per wave
+  __shared__ float s_acc[kManyWaves][D];
+  const int hq = blockIdx.x;
+  const int b = blockIdx.y;
+  const int wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int G = a.group;
+  const int h = hq / G;
+  const int g = hq - h * G;
+  const int64_t base = (int64_t(b) * a.num_kv_heads + h) * a.max_parts;
+  const float* lp = a.part_lse + base * G + g;                    // piece p at lp[p * G]
+  const float* op = a.part_o + (base * G + g) * D + lane * EPL;   // piece p at op[p * G * D]
+  const int nparts = min(a.req_nparts[b], a.max_parts);
+  if (nparts == 1) return;  // (uniform) written by the streaming kernel
+  // Every wave finds the maximum and the sum of the weights over all pieces.
+  float mx = -INFINITY;
+  for (int p = lane; p < nparts; p += 64) mx = fmaxf(mx, lp[int64_t(p) * G]);
+  mx = wave_max(mx);
+  float acc[EPL];
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
+  float S = 0.f;
+  if (mx != -INFINITY) {
+    for (int q0 = 0; q0 < nparts; q0 += 64) {
+      const float w = q0 + lane < nparts ? fast_exp2(lp[int64_t(q0 + lane) * G] - mx) : 0.f;
+      S += w;
+      const int cnt = min(64, nparts - q0);
+      for (int j0 = wave; j0 < cnt; j0 += kManyWaves * kAhead) {
+        float x[kAhead][EPL];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+          const int j = min(j0 + kManyWaves * i, cnt - 1);  // (past the end: weight 0 below)
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) x[i][e] = op[int64_t(q0 + j) * G * D + e];
+        }
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+          const int j = j0 + kManyWaves * i;
+          if (j < cnt) {  // uniform
+            const float wj = readlane_f(w, j);
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) acc[e] = fmaf(wj, x[i][e], acc[e]);
+          }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) s_acc[wave][lane * EPL + e] = acc[e];
+  __syncthreads();
+  S = wave_sum(S);
+  const bool empty = mx == -INFINITY;  // no pages, or none present: 0 and -inf
+  const float inv = empty ? 0.f : 1.f / S;
+  uint16_t* out = a.out + int64_t(b) * a.out_stride + int64_t(hq) * D;
+  for (int d = threadIdx.x; d < D; d += 64 * kManyWaves) {
+    float o = 0.f;
+#pragma unroll
+    for (int w = 0; w < kManyWaves; ++w) o += s_acc[w][d];
+    out[d] = f32_to_bf16(o * inv);
+  }
+  if (a.lse && threadIdx.x == 0)
+    a.lse[int64_t(b) * a.num_kv_heads * G + hq] = empty ? -INFINITY : (mx + fast_log2(S)) * kLn2;
+}
+
+template <int D>
+void launch_merge(const MergeArgs& m, int num_qo_heads, int batch, hipStream_t s) {
+  const dim3 grid{unsigned(num_qo_heads), unsigned(batch)};
+  if (m.max_parts > kSpecParts)
+    decode_merge_many_kernel<D><<<grid, 64 * kManyWaves, 0, s>>>(m);
+  else
+    decode_merge_kernel<D><<<grid, 64, 0, s>>>(m);
 }
 
 // Segment cuts of the flattened page list [0, total): cut[s] is segment s's
@@ -1571,10 +1640,9 @@ int decode_run(const kvc_decode_schedule* sched, const int32_t* plan, const void
   m.out = a.out;
   m.out_stride = out_batch_stride;
   m.lse = lse;
-  const dim3 mgrid{unsigned(Hq), unsigned(batch)};
-  if (D == 128) decode_merge_kernel<128><<<mgrid, 64, 0, s>>>(m);
-  else if (D == 64) decode_merge_kernel<64><<<mgrid, 64, 0, s>>>(m);
-  else decode_merge_kernel<256><<<mgrid, 64, 0, s>>>(m);
+  if (D == 128) launch_merge<128>(m, Hq, batch, s);
+  else if (D == 64) launch_merge<64>(m, Hq, batch, s);
+  else launch_merge<256>(m, Hq, batch, s);
   KVC_LAUNCH_CHECK();
   return ok();
 }
