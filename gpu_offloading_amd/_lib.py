@@ -126,6 +126,10 @@ SIGNATURES = {
         POINTER(KvcDecodeSchedule), _I32P, _P, c_int64, _P, _P, c_int64, c_int64, c_int64,
         _I32P, _I32P, c_int64, _I32P, _P, c_int64, _P, c_int64, c_float, _P, c_int64, _P,
         c_int64, _P, _P]),
+    "kvc_batch_decode_step_run": (c_int, [
+        POINTER(KvcDecodeSchedule), _I32P, _P, c_int64, _P, _P, c_int64, c_int64, c_int64,
+        _I32P, _I32P, c_int64, _I32P, _P, c_int64, _P, c_int64, c_float, _P, c_int64, _P,
+        c_int64, _P, _P]),
     "kvc_prefill_plan": (c_int, [
         c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,
         POINTER(KvcPrefillSchedule), c_void_p, c_int64]),

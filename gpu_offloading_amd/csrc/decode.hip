@@ -9,7 +9,7 @@
 // src/dense/offload_kv_attn.py:24-39 (done in base 2 here).
 //
 // Decode is a GEMV: every K/V byte feeds only `group` query heads, so the
-// kernels are HBM-bound and run on the VALU (no MFMA).
+// kernels are HBM-bound.
 //
 // Schedule (balanced split-KV, computed on the host by kvc_decode_plan like
 // FlashInfer's plan()): the flattened page list indices[0 .. P) of the whole
@@ -22,18 +22,27 @@
 // straight to the output; otherwise each piece leaves an fp32 partial +
 // log2-sum-exp in the workspace and decode_merge_kernel folds them.
 //
-// head_dim 128 (the reference models) uses decode_lds_kernel<G, HPW>: grid
-// (S, Hkv / HPW), one wave per KV head, HPW = 8 heads per workgroup when the
-// heads divide evenly (else 1).  Every wave serves all `group` query heads of
-// its KV head, so K/V are read from HBM exactly once.  The waves stage each
-// page together: wave w loads 256 consecutive 16-byte chunks of the page's
-// (token row x head slice) image (two whole 2 KB token rows for Mixtral), so
-// the workgroup reads the page's K and V blocks as contiguous runs, into a
-// double-buffered LDS tile; one barrier per page; the next two pages are in
-// flight in two register stages meanwhile.  K/V are loaded with the
-// non-temporal hint (read once; 5.7 -> 6.3 TB/s at 32K contexts).  Tile rows are padded by 16 B,
-// which keeps both read patterns below free of LDS bank conflicts and makes
-// every LDS address a lane base plus an immediate:
+// Three streaming kernels, chosen by the plan; all read K/V from HBM exactly
+// once and serve the `group` query heads of a KV head together:
+//
+//   decode_lds_kernel<G>   head_dim 128, group <= 4, a multiple of 8 KV heads:
+//         one workgroup of 8 waves per (segment, 8 heads), pages staged in LDS
+//         as whole 2 KB token rows;
+//   decode_wave_kernel<G, D>   everything else (head_dim 64 / 256, group 8,
+//         other head counts) and small batches: each wave streams pages of one
+//         head straight into registers, no barrier in its loop;
+//   decode_small_kernel<G>  head_dim 128, requests of at most 16 pages: one
+//         workgroup per (request, KV head), no partials.
+//
+// decode_lds_kernel: the waves stage each page together: wave w loads 256
+// consecutive 16-byte chunks of the page's (token row x head slice) image (two
+// whole 2 KB token rows for Mixtral), so the workgroup reads the page's K and V
+// blocks as contiguous runs, into a double-buffered LDS tile; one barrier per
+// page; the next two pages are in flight in two register stages meanwhile.
+// K/V are loaded with the non-temporal hint (read once; 5.7 -> 6.3 TB/s at 32K
+// contexts).  Tile rows are padded by 16 B, which keeps both read patterns
+// below free of LDS bank conflicts and makes every LDS address a lane base
+// plus an immediate:
 //   q.k : lane (token t, query head g) computes the whole 128-dim dot product
 //         with v_dot2_f32_bf16 from 16 ds_read_b128 of row t (the four lanes
 //         of a token read the same address); no cross-lane reduction;
@@ -43,11 +52,6 @@
 // A wave's page ids are loaded once, one per lane (2 registers: up to 128
 // pages per segment), and broadcast with v_readlane, so no dependent global
 // load sits in the streaming loop.
-//
-// head_dim 64 and 256 use decode_reg_kernel: grid (S, ceil(Hkv / 4)), one
-// wave per KV head, no barrier; K/V stay in registers: lane (row r, column c)
-// holds 16 B of tokens r, r+4, r+8, r+12 and q.k is reduced over the 16 lanes
-// of a DPP row.
 #include "kvc_common.h"
 
 #include <algorithm>
@@ -58,13 +62,12 @@
 namespace kvc {
 namespace {
 
-constexpr int kThreads = 256;          // register kernel workgroup
-constexpr int kWaves = kThreads / 64;  // KV heads per register-kernel workgroup
-constexpr int kPage = 16;              // tokens per page (the engine's page_size)
-constexpr int kTokPerRow = 4;          // register kernel: tokens of a page per 16-lane row
-constexpr int kIdRegs = 2;             // page-id registers per lane
+constexpr int kPage = 16;      // tokens per page (the engine's page_size)
+constexpr int kLdsHeads = 8;   // KV heads per workgroup of the LDS kernel
+constexpr int kIdRegs = 2;     // page-id registers per lane
 constexpr int kMaxSegPages = 64 * kIdRegs;
 constexpr int kReadGroup = 4;  // LDS reads scheduled together
+constexpr float kRescaleLog2 = 8.f;  // lazy-rescale threshold (base 2)
 constexpr float kLn2 = 0.69314718055994530942f;
 constexpr float kLog2e = 1.44269504088896340736f;
 
@@ -91,16 +94,19 @@ struct DecodeArgs {
   uint16_t* out;
   int64_t out_stride;      // elements between requests
   float* lse;              // [batch][Hq] natural log, may be null
-  // Fused append (8 KV heads per workgroup): row b of new_k / new_v is
-  // written as request b's last token before it is attended; null: none.
+  // Fused append: row b of new_k / new_v is written as request b's last token
+  // before it is attended; null: none.
   const uint16_t* new_k;
   const uint16_t* new_v;
   int64_t new_k_stride;    // elements between requests
   int64_t new_v_stride;
+  int32_t heads_per_group; // KV heads per workgroup of the wave kernel
+  int32_t q_splits;        // workgroups that share a KV head's query heads
 };
 
-// Pieces, counted from a segment's first, within which a fused append's
-// request may end (the plan reports the most any segment needs).
+// Pieces, counted from a segment's first, within which a request's end may lie
+// for the LDS kernel's fused append (the plan reports the most any segment
+// needs).
 constexpr int kNewMax = 4;
 
 // Compiler-level ordering point for LDS traffic between lanes of one wave
@@ -225,14 +231,15 @@ struct BlockTile {
   uint4 v[kPage * kRowChunks];
 };
 
-// Workgroup = HPW waves = HPW neighbouring KV heads of one segment.  The
-// waves stage each page together: wave w loads 256 consecutive 16-byte chunks
+// Workgroup = 8 waves = 8 neighbouring KV heads of one segment.  The waves
+// stage each page together: wave w loads 256 consecutive 16-byte chunks
 // of the page's (token row x head slice) image, so the workgroup reads the
 // block's rows as long contiguous runs (2 KB per token row for 8 heads), into
 // a double-buffered tile; one barrier per page; then each wave computes its
 // own head from the tile.
-template <int G, int HPW>
-__global__ __launch_bounds__(64 * HPW) void decode_lds_kernel(DecodeArgs a) {
+template <int G>
+__global__ __launch_bounds__(64 * kLdsHeads) void decode_lds_kernel(DecodeArgs a) {
+  constexpr int HPW = kLdsHeads;
   using C = LdsCfg<G>;
   using Tile = BlockTile<HPW>;
   constexpr int D = 128;
@@ -240,9 +247,8 @@ __global__ __launch_bounds__(64 * HPW) void decode_lds_kernel(DecodeArgs a) {
   __shared__ Tile s_tile[2];
   __shared__ float s_p[HPW][kPage * 8];   // softmax weights p[token][query head]
   // Fused append: the new rows (K, V) of the requests that end inside the
-  // segment, by piece index (8 heads per workgroup only).
-  constexpr bool kAppend = HPW == 8;
-  __shared__ uint4 s_new[kAppend ? kNewMax : 1][2][kAppend ? kSliceChunks : 1];
+  // segment, by piece index.
+  __shared__ uint4 s_new[kNewMax][2][kSliceChunks];
 
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
@@ -283,17 +289,17 @@ __global__ __launch_bounds__(64 * HPW) void decode_lds_kernel(DecodeArgs a) {
   Piece pc;
   pc.load(a, k);
   const int k0 = k;
-  const bool appending = kAppend && a.new_k != nullptr;
+  const bool appending = a.new_k != nullptr;
   // Thread i < 2 x kSliceChunks loads chunk i % kSliceChunks of the K (or V)
   // slice of each new row; the rows land in s_new after the first pages'
   // loads are issued.
   // The loads are issued on every path (a piece past the segment's last
   // re-reads that one's row), so the compiler's count of loads in flight stays
   // exact and staging s_new does not wait for the first pages' loads.
-  uint4 nrow[kAppend ? kNewMax : 1];
+  uint4 nrow[kNewMax];
 #pragma unroll
-  for (int i = 0; i < (kAppend ? kNewMax : 1); ++i) nrow[i] = make_uint4(0, 0, 0, 0);
-  if constexpr (kAppend) {
+  for (int i = 0; i < kNewMax; ++i) nrow[i] = make_uint4(0, 0, 0, 0);
+  {
     if (appending) {
       const int is_v = (threadIdx.x & (2 * kSliceChunks - 1)) >= kSliceChunks;
       const int cc = threadIdx.x & (kSliceChunks - 1);
@@ -457,7 +463,7 @@ __global__ __launch_bounds__(64 * HPW) void decode_lds_kernel(DecodeArgs a) {
   auto step = [&](int j, Stage& r, int32_t& id, Tile& tile) __attribute__((always_inline)) {
     const int slot = g0 + j;
     const int valid = pc.valid(slot, id, a.num_blocks);
-    if constexpr (kAppend) {
+    {
       // The request's last page: its new token row comes from s_new (the
       // loaded row is stale) and is written to the cache.
       if (appending && slot == pc.req_last && valid > 0 && k - k0 < kNewMax) {
@@ -504,7 +510,7 @@ __global__ __launch_bounds__(64 * HPW) void decode_lds_kernel(DecodeArgs a) {
     idb = ids.at(1);
     issue(rb, safe_id(idb));
   }
-  if constexpr (kAppend) {
+  {
     if (appending) {
       if (threadIdx.x < 2 * kSliceChunks) {
         const int is_v = threadIdx.x >= kSliceChunks;
@@ -778,200 +784,576 @@ __global__ __launch_bounds__(64 * kSmallWaves) void decode_small_kernel(DecodeAr
 }
 
 // ---------------------------------------------------------------------------
-// head_dim 64 / 256: register kernel.
+// Wave streaming kernel (any head_dim, group and head count).
+//
+// Bound by HBM, so built to keep loads in flight and the arithmetic per byte
+// small: K and V go from memory into registers, nothing is staged in LDS, and
+// no barrier sits in the page loop.  A workgroup's waves are its KV heads times
+// TS page shares: wave (head, ts) streams units ts, ts + TS, ... of the
+// segment (a unit is one page, at head_dim 64 two).  One unit is in flight per
+// wave while another is consumed -- K's registers are refilled as soon as q.k
+// has read them, V's after p.v -- and 8 to 16 waves per CU hide the latency.
+// Every K and V load of the wave reads whole token rows (four rows of 256 B at
+// head_dim 128), which the layouts of the 4x4 matrix instructions allow:
+//   q.k : v_mfma_f32_4x4x4_16b_bf16, block b = 16-byte chunk b of a row, rows =
+//         four tokens, columns = four query heads; the blocks (chunks) are
+//         summed with lane swaps and row rotations that leave row c of 16
+//         lanes with four tokens, head l % 4 in lane l.  (The 16x16x32 layout
+//         needs no such sum, but its loads touch 16 rows of 16 B per quarter
+//         wave: 5.95 against 6.84 TB/s of plain reads.)
+//   softmax : each row of 16 lanes keeps its own maximum and sum over its
+//         tokens, so pages need no exchange; the rows meet once per piece.
+//         The rescale is skipped unless a maximum grows by more than 2^8.
+//   p.v : v_mfma_f32_4x4x1_16b_f32 with p in fp32 as it lies in the lanes and
+//         V widened to fp32 (exact): lane l holds eight dims of its row's token
+//         for the four heads.  A group of one multiplies on the VALU instead.
+// At a piece's end the rows' states are merged in the wave, then the TS waves'
+// through LDS with one barrier, and the piece is written.  Uniform plan records
+// come by scalar loads, which the loads in flight do not delay.
+//
+// One layer with its append (start: the kernel it replaces with the merge of
+// its time), us:
+//   32 requests of 500-3001 tokens, 8 KV heads, group 8, head_dim 64: 63.8 -> 32.5
+//   64 of 512-4096, group 8, head_dim 128: 133 -> 101 (5.6 TB/s)
+//   64 of 512-4096, one KV head, group 4, head_dim 128: 35.6 -> 21.0
+//   32 of 500-3000, 8 KV heads, head_dim 256, group 4: 93 -> 80 (5.7 TB/s)
+//   32 of 500-3000, 16 KV heads, head_dim 64, group 1: 47.9 -> 44.8
 // ---------------------------------------------------------------------------
-// Load the D/16 bf16 elements one lane owns (D/32 32-bit words).
-template <int D, bool kStream = false>
-__device__ __forceinline__ void load_slice(uint32_t (&w)[D / 32], const uint16_t* p) {
-  if constexpr (D == 64) {
-    const uint2 x = *reinterpret_cast<const uint2*>(p);
-    w[0] = x.x; w[1] = x.y;
-  } else {
-    static_assert(D == 128 || D == 256, "head_dim must be 64, 128 or 256");
-#pragma unroll
-    for (int i = 0; i < D / 128; ++i) {
-      const uint4 x = kStream ? load_stream(reinterpret_cast<const uint4*>(p) + i)
-                              : reinterpret_cast<const uint4*>(p)[i];
-      w[4 * i + 0] = x.x; w[4 * i + 1] = x.y; w[4 * i + 2] = x.z; w[4 * i + 3] = x.w;
-    }
-  }
-}
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
+// Vectors at the element alignment the callers guarantee (head_dim 64 takes
+// 8-byte aligned rows, the output 4-byte aligned ones); gfx950 moves them with
+// one dwordx4 all the same.
+typedef u32x4_t u32x4_a8_t __attribute__((aligned(8)));
+typedef u32x4_t u32x4_a4_t __attribute__((aligned(4)));
 
-template <int D>
-struct PageRegs {
-  uint32_t k[kTokPerRow][D / 32];
-  uint32_t v[kTokPerRow][D / 32];
+// Word 3 of a raw buffer resource (32-bit data, no swizzle; loads past
+// num_records return zeros) and the non-temporal bit of a buffer load.
+constexpr int kBufferRsrcWord3 = 0x00020000;
+constexpr int kNonTemporal = 2;
+
+// G: query heads of a KV head that one workgroup serves.  At head_dim 256 a
+// group of 8 is served as two workgroups of four (q_splits 2): its accumulators
+// alone would fill a wave's registers.
+template <int G, int D>
+struct WaveCfg {
+  static_assert(G <= 4 || D < 256, "four query heads per wave at head_dim 256");
+  // Waves per workgroup: as many as a CU's registers hold.
+  static constexpr int kWaves =
+      G == 1 ? (D == 256 ? 12 : 16) : (D == 256 ? 8 : 12);
+  static constexpr int kPages = D == 64 && G < 8 ? 2 : 1;  // pages a wave takes at a time
+  static constexpr int kGroups = G == 8 ? 2 : 1;   // query heads in fours
+  static constexpr int kGroupHeads = G < 4 ? G : 4;
+  static constexpr int kLoads = D / 32;            // 16-byte K (and V) loads per lane and page
+  static constexpr int kQ = D == 256 ? 2 : 1;      // 16-byte q chunks per lane and group
+  static constexpr int kDims = D == 256 ? 16 : 8;  // output dims per lane
 };
 
-template <int D>
-__device__ __forceinline__ void load_page_regs(const DecodeArgs& a, PageRegs<D>& r,
-                                               int32_t blk, int64_t lane_off) {
-  const int64_t base = int64_t(blk) * a.block_stride + lane_off;
-#pragma unroll
-  for (int j = 0; j < kTokPerRow; ++j)
-    load_slice<D, true>(r.k[j], a.k_cache + base + int64_t(j) * kTokPerRow * a.token_stride);
-#pragma unroll
-  for (int j = 0; j < kTokPerRow; ++j)
-    load_slice<D, true>(r.v[j], a.v_cache + base + int64_t(j) * kTokPerRow * a.token_stride);
+// x and y summed over the wave's halves: lanes < 32 get x's sum, the others y's.
+__device__ __forceinline__ float swap32_add(float x, float y) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// x and y summed over pairs of 16-lane rows (0 + 1, 2 + 3): even rows get x's
+// sum, odd rows y's.
+__device__ __forceinline__ float swap16_add(float x, float y) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// D += A B over 16 blocks of four lanes: A row l % 4 and B column l % 4 of
+// block l / 4, four bf16 each (a0, a1 / b0, b1); D register r: row r, column l % 4.
+__device__ __forceinline__ f32x4_t mfma_4x4x4(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1,
+                                              f32x4_t d) {
+  return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(
+      __builtin_bit_cast(i16x4_t, (uint64_t(a1) << 32) | a0),
+      __builtin_bit_cast(i16x4_t, (uint64_t(b1) << 32) | b0), d, 0, 0, 0);
 }
 
-// Fold one page into the row's online-softmax state.
+// Eight output dims (from d0) of a finished piece for query head h * group + g.
+template <int D>
+__device__ __forceinline__ void write_dims8(const DecodeArgs& a, const int4& pc, int h, int group,
+                                            int g, int d0, const float* o) {
+  const int hq = h * group + g;
+  if (pc.w < 0) {
+    u32x4_t w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      w[e] = uint32_t(f32_to_bf16(o[2 * e])) | (uint32_t(f32_to_bf16(o[2 * e + 1])) << 16);
+    *reinterpret_cast<u32x4_a4_t*>(a.out + int64_t(pc.x) * a.out_stride + int64_t(hq) * D + d0) = w;
+  } else {
+    const int64_t pr = ((int64_t(pc.x) * a.num_kv_heads + h) * a.max_parts + pc.w) * group + g;
+    float4* dst = reinterpret_cast<float4*>(a.part_o + pr * D + d0);
+    dst[0] = make_float4(o[0], o[1], o[2], o[3]);
+    dst[1] = make_float4(o[4], o[5], o[6], o[7]);
+  }
+}
+__device__ __forceinline__ void write_lse(const DecodeArgs& a, const int4& pc, int h, int group,
+                                          int g, float lse2) {
+  const int hq = h * group + g;
+  if (pc.w < 0) {
+    if (a.lse) a.lse[int64_t(pc.x) * a.num_kv_heads * group + hq] = lse2 * kLn2;
+  } else {
+    a.part_lse[((int64_t(pc.x) * a.num_kv_heads + h) * a.max_parts + pc.w) * group + g] = lse2;
+  }
+}
+
+// A uniform int4 of the plan image as a scalar load: waiting for it does not
+// wait for the page loads in flight (those are counted apart).
+__device__ __forceinline__ int4 scalar_int4(const int4* p, int i) {
+  typedef int i32x4_t __attribute__((ext_vector_type(4)));
+  typedef const __attribute__((address_space(4))) i32x4_t* cptr;
+  const i32x4_t v = ((cptr)(uintptr_t)(p))[i];
+  return make_int4(v[0], v[1], v[2], v[3]);
+}
+
+// Workgroup barrier that orders LDS traffic only: global loads stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The lane index as a value that what is computed from it cannot be hoisted
+// past: the rare paths of a loop then hold no registers through it.
+__device__ __forceinline__ int local_lane() {
+  int l = threadIdx.x & 63;
+  asm volatile("" : "+v"(l));
+  return l;
+}
+
+// Value of lane 4 (l / 4) + V for every lane l.
+template <int V>
+__device__ __forceinline__ float quad_lane(float x) {
+  return dpp<V * 0x55>(x);
+}
+
 template <int G, int D>
-__device__ __forceinline__ void consume_page_regs(const uint32_t (&qw)[G][D / 32],
-                                                  PageRegs<D>& r, int valid, int row,
-                                                  float scale_log2, float (&m)[G],
-                                                  float (&l)[G], float (&acc)[G][D / 16]) {
-  constexpr int W = D / 32;
-  if (valid < kPage) {
+__global__ __launch_bounds__((64 * WaveCfg<G, D>::kWaves), (WaveCfg<G, D>::kWaves / 4)) void decode_wave_kernel(DecodeArgs a) {
+  using C = WaveCfg<G, D>;
+  constexpr int W = C::kWaves, NG = C::kGroups, NL = C::kLoads, NE = C::kDims, PU = C::kPages;
+  __shared__ float s_o[2][W][G][D];
+  __shared__ float s_m[2][W][G], s_l[2][W][G];
+
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int hpw = a.heads_per_group;
+  const int hw = wave % hpw, ts = wave / hpw, TS = W / hpw;
+  const int split = blockIdx.y % a.q_splits, h0 = blockIdx.y / a.q_splits * hpw;
+  const int h = h0 + hw;
+  const int group = G * a.q_splits;  // query heads of a KV head
+  const int4 segment = scalar_int4(a.segments, blockIdx.x);
+  int k = segment.x;
+  const int k_end = segment.y, g0 = segment.z, n = segment.w;
+  if (k >= k_end) return;  // uniform over the workgroup
+
+  // Lane roles.  K (and q.k): row of four consecutive tokens l % 4, 16-byte
+  // chunk l / 4.  V (and p.v): tokens t_row .. t_row + 3 of the page, chunk
+  // l % 16.
+  const int c = lane >> 4, nn = lane & 15;
+  const int t_row = D == 64 ? 8 * (c & 1) + 4 * (c >> 1) : 4 * c;
+  const uint32_t tsb = uint32_t(a.token_stride * 2);
+  const int k_chunk = D == 64 ? (lane >> 2) & 7 : lane >> 2;
+  const int k_tok = (D == 64 ? 4 * (lane >> 5) : 0) + (lane & 3);
+  const int v_chunk = D == 64 ? nn & 7 : nn;
+  const int v_tok = t_row + (D == 64 ? nn >> 3 : 0);
+  // Byte offset of load u inside a page block (head_dim 256's second half is
+  // 256 bytes further), and its token.
+  constexpr int NT = NL < 4 ? NL : 4;
+  uint32_t k_off[NT], v_off[NT];
+  auto k_step = [](int u) { return D == 64 ? 8 * u : 4 * (u & 3); };
+  auto v_step = [](int u) { return D == 64 ? 2 * u : u & 3; };
+  auto d_step = [](int u) { return D == 256 ? (u >> 2) * 256 : 0; };
 #pragma unroll
-    for (int j = 0; j < kTokPerRow; ++j)
-      if (row + kTokPerRow * j >= valid)
-#pragma unroll
-        for (int w = 0; w < W; ++w) r.v[j][w] = 0u;
+  for (int u = 0; u < NT; ++u) {
+    k_off[u] = uint32_t(k_tok + k_step(u)) * tsb + uint32_t(h * D * 2 + k_chunk * 16);
+    v_off[u] = uint32_t(v_tok + v_step(u)) * tsb + uint32_t(h * D * 2 + v_chunk * 16);
   }
-  float s[kTokPerRow][G];
+  const char* kbytes = reinterpret_cast<const char*>(a.k_cache);
+  const char* vbytes = reinterpret_cast<const char*>(a.v_cache);
+  const int64_t block_bytes = a.block_stride * 2;
+
+  // This wave's units of PU consecutive pages: unit ts, ts + TS, ... of the
+  // segment; the pages' ids one per lane.
+  const int nw = n > PU * ts ? (n - PU * ts + PU * TS - 1) / (PU * TS) : 0;
+  auto page_slot = [&](int j, int x) { return g0 + PU * (ts + TS * j) + x; };
+  int32_t idr[kIdRegs];
+  {
+    const int64_t last = a.num_indices - 1;
 #pragma unroll
-  for (int j = 0; j < kTokPerRow; ++j)
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      float d = 0.f;
-#pragma unroll
-      for (int w = 0; w < W; ++w) d = dot2_bf16(qw[g][w], r.k[j][w], d);
-      d = row16_sum(d) * scale_log2;
-      s[j][g] = row + kTokPerRow * j < valid ? d : kNegBig;
-    }
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    float mx = s[0][g];
-#pragma unroll
-    for (int j = 1; j < kTokPerRow; ++j) mx = fmaxf(mx, s[j][g]);
-    const float m_new = fmaxf(m[g], mx);
-    const float alpha = fast_exp2(m[g] - m_new);
-    float psum = 0.f;
-#pragma unroll
-    for (int j = 0; j < kTokPerRow; ++j) {
-      s[j][g] = row + kTokPerRow * j < valid ? fast_exp2(s[j][g] - m_new) : 0.f;
-      psum += s[j][g];
-    }
-    l[g] = fmaf(l[g], alpha, psum);
-    m[g] = m_new;
-#pragma unroll
-    for (int e = 0; e < D / 16; ++e) acc[g][e] *= alpha;
-  }
-#pragma unroll
-  for (int j = 0; j < kTokPerRow; ++j)
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-      const float v0 = bf16lo(r.v[j][w]);
-      const float v1 = bf16hi(r.v[j][w]);
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        acc[g][2 * w] = fmaf(s[j][g], v0, acc[g][2 * w]);
-        acc[g][2 * w + 1] = fmaf(s[j][g], v1, acc[g][2 * w + 1]);
+    for (int i = 0; i < kIdRegs; ++i) {
+      idr[i] = -1;
+      if (64 * i < PU * nw) {
+        const int j = lane + 64 * i;
+        const int64_t slot = page_slot(j / PU, j % PU);
+        const int32_t v = a.indices[min(slot, last)];
+        idr[i] = (slot < g0 + n && slot <= last) ? v : -1;
       }
     }
-}
-
-template <int G, int D>
-__global__ __launch_bounds__(kThreads) void decode_reg_kernel(DecodeArgs a) {
-  constexpr int W = D / 32;
-  constexpr int E = D / 16;
-  const int wave = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  const int h = blockIdx.y * kWaves + wave;
-  if (h >= a.num_kv_heads) return;
-  const int4 segment = a.segments[blockIdx.x];
-  int g0, n;
-  segment_span(segment, g0, n);
-  int k = segment.x;
-  const int k_end = segment.y;
-  if (k >= k_end || n <= 0) return;
-  const int row = lane >> 4;
-  const int col = lane & 15;
-  const int64_t lane_off = int64_t(row) * a.token_stride + int64_t(h) * D + col * E;
-
-  SegmentIds ids;
-  ids.load(a, g0, n, lane);
-  Piece pc;
-  pc.load(a, k);
-
-  uint32_t qw[G][W];
-  auto load_q = [&](int b) __attribute__((always_inline)) {
-    const uint16_t* qb = a.q + int64_t(b) * a.q_stride + int64_t(h) * G * D + col * E;
+  }
+  auto id_at = [&](int j) __attribute__((always_inline)) {
+    int32_t v = __builtin_amdgcn_readlane(idr[0], j & 63);
 #pragma unroll
-    for (int g = 0; g < G; ++g) load_slice<D>(qw[g], qb + g * D);
+    for (int i = 1; i < kIdRegs; ++i) {
+      const int32_t x = __builtin_amdgcn_readlane(idr[i], j & 63);
+      v = (j >> 6) == i ? x : v;
+    }
+    return v;
   };
-  float m[G], l[G], acc[G][E];
+
+  int4 cp = scalar_int4(a.pieces, 2 * k), ct = scalar_int4(a.pieces, 2 * k + 1);
+  // The piece of the next page to be requested.
+  int ki = k;
+  int4 ip = cp, it = ct;
+  // q: head l % 4 of each four, the 16-byte chunk(s) of this lane's K loads.
+  const int q_head = (lane & 3) % C::kGroupHeads;
+  const uint32_t q_off = uint32_t((h * group + G * split + q_head) * D + k_chunk * 8) * 2;
+  const int page_bytes = kPage * int(tsb);  // under 2 GiB (host check)
+  u32x4_t q[NG][C::kQ], qn[NG][C::kQ];  // of the current piece and the next
+  auto load_q = [&](u32x4_t (&dst)[NG][C::kQ], int b) __attribute__((always_inline)) {
+    const char* qb = reinterpret_cast<const char*>(a.q + int64_t(b) * a.q_stride);
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int x = 0; x < C::kQ; ++x)
+        dst[g][x] = *reinterpret_cast<const u32x4_a8_t*>(qb + (4 * g * D + 128 * x) * 2 + q_off);
+  };
+
+  // The unit in the K and V registers: K's next unit is requested once q.k has
+  // read them, V's after p.v, so one set of registers keeps a unit in flight.
+  // A missing page, or one past the segment's last, loads nothing.
+  struct Ids {
+    int32_t v[PU];
+  };
+  u32x4_t kr[PU][NL], vr[PU][NL];
+  auto unit_ids = [&](int j) __attribute__((always_inline)) {
+    Ids r;
+#pragma unroll
+    for (int x = 0; x < PU; ++x) {
+      const int32_t id = j < nw ? id_at(PU * j + x) : -1;
+      r.v[x] = id < a.num_blocks ? id : -1;
+    }
+    return r;
+  };
+  auto load_unit = [&](u32x4_t (&dst)[PU][NL], const char* base, const uint32_t (&off)[NT],
+                       const Ids& ids) __attribute__((always_inline)) {
+#pragma unroll
+    for (int x = 0; x < PU; ++x) {
+      const int32_t id = ids.v[x];
+      const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<char*>(base + int64_t(max(id, 0)) * block_bytes), 0, id < 0 ? 0 : page_bytes,
+          kBufferRsrcWord3);
+#pragma unroll
+      for (int u = 0; u < NL; ++u)
+        dst[x][u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, int(off[u & 3]) + d_step(u), 0,
+                                                          kNonTemporal);
+    }
+  };
+
+  float m[NG], l[NG];
+  // acc[g][e]: this lane's dim e for the four query heads of g (G 1: one head).
+  constexpr int NH = G == 1 ? 1 : 4;
+  typedef float acc_t __attribute__((ext_vector_type(NH)));
+  acc_t acc[NG][NE];
   auto reset = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
+    for (int g = 0; g < NG; ++g) {
       m[g] = kNegBig;
       l[g] = 0.f;
 #pragma unroll
-      for (int e = 0; e < E; ++e) acc[g][e] = 0.f;
+      for (int e = 0; e < NE; ++e) acc[g][e] = 0.f;
     }
   };
-  auto finalize = [&]() __attribute__((always_inline)) {
-    // Merge the four rows (lanes c, c+16, c+32, c+48 hold the same dims).
+
+  int parity = 0;
+  // Close piece k: the four rows' states of every wave are merged, then (TS > 1)
+  // those of the waves that shared the piece, and the piece is written.
+  auto finish = [&]() __attribute__((always_inline)) {
+    const int fl = local_lane();
+    const int c = fl >> 4, nn = fl & 15, v_chunk = D == 64 ? nn & 7 : nn;
 #pragma unroll
-    for (int off = 16; off <= 32; off <<= 1) {
+    for (int g = 0; g < NG; ++g) {
+      float M = fmaxf(m[g], __shfl_xor(m[g], 16));
+      M = fmaxf(M, __shfl_xor(M, 32));
+      const float w = fast_exp2(m[g] - M);
+      float L = l[g] * w;
+      L += __shfl_xor(L, 16);
+      L += __shfl_xor(L, 32);
+      const float w0 = quad_lane<0>(w), w1 = quad_lane<1>(w), w2 = quad_lane<2>(w),
+                  w3 = quad_lane<3>(w);
+      // Row c ends up with head c: swap halves, then odd and even rows.
+      float o[NE];
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const float mo = __shfl_xor(m[g], off);
-        const float lo = __shfl_xor(l[g], off);
-        const float mm = fmaxf(m[g], mo);
-        const float wa = fast_exp2(m[g] - mm);
-        const float wb = fast_exp2(mo - mm);
-        l[g] = l[g] * wa + lo * wb;
-        m[g] = mm;
+      for (int e = 0; e < NE; ++e) {
+        float x0 = acc[g][e][0] * w0, x1 = acc[g][e][1 % NH] * w1;
+        float x2 = acc[g][e][2 % NH] * w2, x3 = acc[g][e][3 % NH] * w3;
+        if constexpr (D == 64) {
+          x0 += dpp<kDppRowRor8>(x0);
+          x1 += dpp<kDppRowRor8>(x1);
+          x2 += dpp<kDppRowRor8>(x2);
+          x3 += dpp<kDppRowRor8>(x3);
+        }
+        o[e] = swap16_add(swap32_add(x0, x2), swap32_add(x1, x3));
+      }
+      const float Lc = __shfl(L, c), Mc = __shfl(M, c);
+      const int gl = 4 * g + c, gq = G * split + gl;  // query head of the workgroup, of the KV head
+      if (TS == 1) {
+        if (c < C::kGroupHeads) {
+          const float inv = Lc > 0.f ? 1.f / Lc : 0.f;
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const float ao = __shfl_xor(acc[g][e], off);
-          acc[g][e] = acc[g][e] * wa + ao * wb;
+          for (int e = 0; e < NE; ++e) o[e] *= inv;
+          if (D != 64 || nn < 8) {
+#pragma unroll
+            for (int x = 0; x < NE / 8; ++x)
+              write_dims8<D>(a, cp, h, group, gq, 128 * x + 8 * v_chunk, o + 8 * x);
+          }
+          if (nn == 0) write_lse(a, cp, h, group, gq, Lc > 0.f ? Mc + fast_log2(Lc) : -INFINITY);
+        }
+      } else if (c < C::kGroupHeads) {
+        if (D != 64 || nn < 8) {
+#pragma unroll
+          for (int x = 0; x < NE / 8; ++x) {
+            float4* dst = reinterpret_cast<float4*>(&s_o[parity][wave][gl][128 * x + 8 * v_chunk]);
+            dst[0] = make_float4(o[8 * x], o[8 * x + 1], o[8 * x + 2], o[8 * x + 3]);
+            dst[1] = make_float4(o[8 * x + 4], o[8 * x + 5], o[8 * x + 6], o[8 * x + 7]);
+          }
+        }
+        if (nn == 0) {
+          s_m[parity][wave][gl] = Mc;
+          s_l[parity][wave][gl] = Lc;
         }
       }
     }
-    if (row == 0) {
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const float inv = l[g] > 0.f ? 1.f / l[g] : 0.f;
-        float o[E];
-#pragma unroll
-        for (int e = 0; e < E; ++e) o[e] = acc[g][e] * inv;
-        write_piece<D, E>(a, pc.desc, h, G, g, col * E, o,
-                          l[g] > 0.f ? m[g] + fast_log2(l[g]) : -INFINITY, col == 0);
+    if (TS > 1) {
+      // One barrier per piece: the other parity's buffers are only written
+      // again after the next piece's barrier.
+      lds_barrier();
+      for (int i = 64 * wave + fl; i < hpw * G * (D / 2); i += 64 * W) {
+        const int d = 2 * (i % (D / 2)), r = i / (D / 2);
+        const int gq = r % G, hh = r / G;
+        float M = kNegBig;
+        for (int t = 0; t < TS; ++t) M = fmaxf(M, s_m[parity][hh + hpw * t][gq]);
+        float L = 0.f, o0 = 0.f, o1 = 0.f;
+        for (int t = 0; t < TS; ++t) {
+          const int ww = hh + hpw * t;
+          const float w = fast_exp2(s_m[parity][ww][gq] - M);
+          L = fmaf(s_l[parity][ww][gq], w, L);
+          const float2 x = *reinterpret_cast<const float2*>(&s_o[parity][ww][gq][d]);
+          o0 = fmaf(x.x, w, o0);
+          o1 = fmaf(x.y, w, o1);
+        }
+        const float inv = L > 0.f ? 1.f / L : 0.f;
+        const float o[2] = {o0 * inv, o1 * inv};
+        write_piece<D, 2>(a, cp, h0 + hh, group, G * split + gq, d, o,
+                          L > 0.f ? M + fast_log2(L) : -INFINITY, d == 0);
       }
+      parity ^= 1;
     }
   };
 
-  // Two register sets: page j is consumed while page j+1 is in flight.
-  auto safe = [&](int32_t id) __attribute__((always_inline)) { return (id >= 0 && id < a.num_blocks) ? id : 0; };
-  PageRegs<D> ra, rb;
-  auto step = [&](int j, PageRegs<D>& cur, int32_t id, PageRegs<D>& nxt, int32_t& nid) __attribute__((always_inline)) {
-    const int slot = g0 + j;
-    if (j + 1 < n) {
-      nid = ids.at(j + 1);
-      load_page_regs<D>(a, nxt, safe(nid), lane_off);
-    }
-    consume_page_regs<G, D>(qw, cur, pc.valid(slot, id, a.num_blocks), row, a.scale_log2,
-                            m, l, acc);
-    if (slot + 1 == pc.desc.z) {
-      finalize();
-      if (++k < k_end) {
-        pc.load(a, k);
-        load_q(pc.desc.x);
-        reset();
+  // Fused append.  The wave that owns a request's last page writes the new
+  // token's row of its head just before it requests the page: one wave's memory
+  // operations are performed in order, so the page comes back with the row.
+  // Lane l holds 16-byte chunk l % (D / 8) of the K (or V) row; the row of the
+  // first such page among the segment's leading pieces is loaded ahead.
+  const bool appending = a.new_k != nullptr;
+  auto load_new = [&](int b) __attribute__((always_inline)) {
+    const int nl = local_lane();
+    const uint16_t* src = nl >= D / 8 ? a.new_v + int64_t(b) * a.new_v_stride
+                                      : a.new_k + int64_t(b) * a.new_k_stride;
+    u32x4_t r = {0, 0, 0, 0};
+    if (nl < D / 4) r = *reinterpret_cast<const u32x4_a4_t*>(src + h * D + (nl % (D / 8)) * 8);
+    return r;
+  };
+  u32x4_t nrow = {0, 0, 0, 0};
+  int nslot = -1;
+  if (appending) {
+    for (int i = 0; i < kNewMax && k + i < k_end && nslot < 0; ++i) {
+      const int4 pd = scalar_int4(a.pieces, 2 * (k + i)), pt = scalar_int4(a.pieces, 2 * (k + i) + 1);
+      if (pd.z == pt.x + 1 && (pt.x - g0) / PU % TS == ts) {
+        nslot = pt.x;
+        nrow = load_new(pd.x);
       }
     }
+  }
+  auto append_page = [&](int slot, int32_t id) __attribute__((always_inline)) {
+    if (id < 0) return;
+    while (slot >= ip.z && ki + 1 < k_end) {
+      ++ki;
+      ip = scalar_int4(a.pieces, 2 * ki);
+      it = scalar_int4(a.pieces, 2 * ki + 1);
+    }
+    const int tnew = min(max(it.y, 0), kPage) - 1;
+    if (slot != it.x || tnew < 0) return;
+    if (slot != nslot) nrow = load_new(ip.x);
+    const int nl = local_lane();
+    const char* dst = (nl >= D / 8 ? vbytes : kbytes) + int64_t(id) * block_bytes +
+                      int64_t(tnew) * tsb + h * D * 2 + (nl % (D / 8)) * 16;
+    if (nl < D / 4)
+      __builtin_nontemporal_store(nrow, reinterpret_cast<u32x4_a8_t*>(const_cast<char*>(dst)));
+    wave_lds_fence();
   };
 
-  load_q(pc.desc.x);
+  auto append_unit = [&](int j, const Ids& ids) __attribute__((always_inline)) {
+#pragma unroll
+    for (int x = 0; x < PU; ++x) append_page(page_slot(j, x), ids.v[x]);
+  };
+
+  Ids id = unit_ids(0);
+  if (appending) append_unit(0, id);
+  load_unit(kr, kbytes, k_off, id);
+  load_unit(vr, vbytes, v_off, id);
+  load_q(q, cp.x);
+  load_q(qn, scalar_int4(a.pieces, 2 * min(k + 1, k_end - 1)).x);
   reset();
-  int32_t ida = ids.at(0), idb = 0;
-  load_page_regs<D>(a, ra, safe(ida), lane_off);
-  for (int j = 0; j < n; j += 2) {
-    step(j, ra, ida, rb, idb);
-    if (j + 1 < n) step(j + 1, rb, idb, ra, ida);
+  int pos = nw > 0 ? page_slot(0, 0) : INT32_MAX;  // first page not yet consumed
+  for (int j = 0;;) {
+    while (pos >= cp.z) {
+      finish();
+      if (++k >= k_end) return;
+      cp = scalar_int4(a.pieces, 2 * k);
+      ct = scalar_int4(a.pieces, 2 * k + 1);
+#pragma unroll
+      for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int x = 0; x < C::kQ; ++x) q[g][x] = qn[g][x];
+      load_q(qn, scalar_int4(a.pieces, 2 * min(k + 1, k_end - 1)).x);
+      reset();
+    }
+    // The tokens of each page that the piece holds: none of a missing page, or
+    // of one that lies in another piece (a unit may cross into the next piece:
+    // it is then consumed once for each, and refilled after the last).
+    int valid[PU];
+#pragma unroll
+    for (int x = 0; x < PU; ++x) {
+      const int slot = page_slot(j, x);
+      const bool in = PU == 1 || (slot >= pos && slot < cp.z);
+      valid[x] = id.v[x] < 0 || !in ? 0 : (slot == ct.x ? min(max(ct.y, 0), kPage) : kPage);
+    }
+    const bool crosses = PU > 1 && page_slot(j, PU - 1) >= cp.z && cp.z < g0 + n;  // uniform
+    const Ids next = unit_ids(j + 1);
+    float p[NG][PU][4];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+#pragma unroll
+      for (int y = 0; y < PU; ++y) {
+        f32x4_t d[NT];
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+          d[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int x = 0; x < C::kQ; ++x) {
+            const u32x4_t kk = kr[y][i + 4 * x], qq = q[g][x];
+            d[i] = mfma_4x4x4(kk[0], kk[1], qq[0], qq[1], d[i]);
+            d[i] = mfma_4x4x4(kk[2], kk[3], qq[2], qq[3], d[i]);
+          }
+        }
+        // Sum over the chunks of a row; lane row c keeps tokens t_row .. +3.
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float x;
+          if constexpr (D == 64)
+            x = swap16_add(d[0][r], d[1][r]);
+          else
+            x = swap16_add(swap32_add(d[0][r], d[2][r]), swap32_add(d[1][r], d[3][r]));
+          x += dpp<kDppRowRor4>(x);
+          x += dpp<kDppRowRor8>(x);
+          p[g][y][r] = x;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (!crosses) {
+      if (appending) append_unit(j + 1, next);
+      load_unit(kr, kbytes, k_off, next);
+    }
+#pragma unroll
+    for (int y = 0; y < PU; ++y) {
+      if (valid[y] < kPage) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            p[g][y][r] = t_row + r < valid[y] ? p[g][y][r] : -INFINITY;
+        // Rows past the end may hold anything (even NaN bits): 0 * v stays 0.
+        // (A page without tokens is left out of p.v.)
+        if (PU == 1 || valid[y] > 0) {
+#pragma unroll
+          for (int u = 0; u < NL; ++u)
+            if (v_tok + v_step(u) >= valid[y]) vr[y][u] = u32x4_t{0, 0, 0, 0};
+        }
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int y = 0; y < PU; ++y)
+        mx = fmaxf(mx, fmaxf(fmaxf(p[g][y][0], p[g][y][1]), fmaxf(p[g][y][2], p[g][y][3])));
+      const float cand = fmaxf(m[g], mx * a.scale_log2);
+      const bool grow = cand > m[g] + kRescaleLog2;
+      if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+        const float al = grow ? fast_exp2(m[g] - cand) : 1.f;
+        m[g] = grow ? cand : m[g];
+        l[g] *= al;
+        const float a0 = quad_lane<0>(al), a1 = quad_lane<1>(al), a2 = quad_lane<2>(al),
+                    a3 = quad_lane<3>(al);
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+          acc[g][e][0] *= a0;
+          if constexpr (G > 1) {
+            acc[g][e][1] *= a1;
+            acc[g][e][2] *= a2;
+            acc[g][e][3] *= a3;
+          }
+        }
+      }
+#pragma unroll
+      for (int y = 0; y < PU; ++y) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          p[g][y][r] = fast_exp2(fmaf(p[g][y][r], a.scale_log2, -m[g]));
+        l[g] += (p[g][y][0] + p[g][y][1]) + (p[g][y][2] + p[g][y][3]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < PU * NL; ++i) {
+      const int y = i / NL, u = i % NL;
+      if (PU > 1 && valid[y] == 0) continue;  // uniform
+      float pu[NG];
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        if constexpr (D == 64)
+          pu[g] = nn < 8 ? p[g][y][2 * u] : p[g][y][2 * u + 1];
+        else
+          pu[g] = p[g][y][u & 3];
+      }
+      const int e0 = D == 256 ? 8 * (u >> 2) : 0;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float v0 = bf16lo(vr[y][u][w]), v1 = bf16hi(vr[y][u][w]);
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+          if constexpr (G == 1) {
+            acc[g][e0 + 2 * w][0] = fmaf(pu[g], v0, acc[g][e0 + 2 * w][0]);
+            acc[g][e0 + 2 * w + 1][0] = fmaf(pu[g], v1, acc[g][e0 + 2 * w + 1][0]);
+          } else {
+            acc[g][e0 + 2 * w] =
+                __builtin_amdgcn_mfma_f32_4x4x1f32(pu[g], v0, acc[g][e0 + 2 * w], 0, 0, 0);
+            acc[g][e0 + 2 * w + 1] =
+                __builtin_amdgcn_mfma_f32_4x4x1f32(pu[g], v1, acc[g][e0 + 2 * w + 1], 0, 0, 0);
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);  // (bounds the widened V held at once)
+    }
+    if (!crosses) {
+      load_unit(vr, vbytes, v_off, next);
+      id = next;
+      ++j;
+      pos = j < nw ? page_slot(j, 0) : INT32_MAX;
+    } else {
+      pos = cp.z;
+    }
   }
 }
 
@@ -1003,10 +1385,10 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 
 // One wave per (request, query head), for plans with at most kSpecParts pieces
-// per request.  The partials and the log2-sum-exps are loaded together with
-// the request's piece count (all inside the max_parts rows the workspace holds
-// for the request), so a merge costs one memory round trip; lane p weighs
-// piece p and every lane folds its D/64 dims.  Requests with a single piece were finished
+// per request.  The partials and the log2-sum-exps are loaded together with the request's piece
+// count (all inside the max_parts rows the workspace holds for the request),
+// so the common case costs one memory round trip; lane p weighs piece p and
+// every lane folds its D/64 dims.  Requests with a single piece were finished
 // by the streaming kernel; requests with no pages get a zero output and
 // lse = -inf.
 //
@@ -1076,12 +1458,11 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(MergeArgs a) {
 // Plans whose requests may have more than kSpecParts pieces (few requests over
 // many segments): the same merge by four waves per (request, query head), wave
 // w folding pieces w, w + 4, ... with four partials in flight, the waves' sums
-// added through LDS.  Bound by latency: one wave alone folded them as a chain
-// of single loads, 15.7 us of a 28.1 us decode at 65 pieces (8 requests of
-// 300-2000 tokens, 8 KV heads; 18.3 us this way), and a decode of one request
-// of 4096 tokens (256 pieces) took 70.2 us against 25.2.  At 16 pieces and
-// fewer one wave's loads are already a single batch and its workgroup, with no
-// barrier, starts and ends sooner.
+// added through LDS.  One wave alone folds them as a chain of single loads:
+// 15.7 us at 65 pieces (8 requests of 300-2000 tokens, 8 KV heads) and 57 us
+// at 256 (one request of 4096), against 5.1 and 9.1 us this way.  At 16 pieces
+// and fewer the chain is already one batch of loads and the smaller workgroup
+// starts sooner.
 constexpr int kManyWaves = 4;
 
 template <int D>
@@ -1138,8 +1519,7 @@ __global__ __launch_bounds__(64 * kManyWaves) void decode_merge_many_kernel(Merg
   for (int e = 0; e < EPL; ++e) s_acc[wave][lane * EPL + e] = acc[e];
   __syncthreads();
   S = wave_sum(S);
-  const bool empty = mx == -INFINITY;  // no pages, or none present: 0 and -inf
-  const float inv = empty ? 0.f : 1.f / S;
+  const float inv = S > 0.f ? 1.f / S : 0.f;  // no pages, or none present: 0 and -inf
   uint16_t* out = a.out + int64_t(b) * a.out_stride + int64_t(hq) * D;
   for (int d = threadIdx.x; d < D; d += 64 * kManyWaves) {
     float o = 0.f;
@@ -1148,7 +1528,7 @@ __global__ __launch_bounds__(64 * kManyWaves) void decode_merge_many_kernel(Merg
     out[d] = f32_to_bf16(o * inv);
   }
   if (a.lse && threadIdx.x == 0)
-    a.lse[int64_t(b) * a.num_kv_heads * G + hq] = empty ? -INFINITY : (mx + fast_log2(S)) * kLn2;
+    a.lse[int64_t(b) * a.num_kv_heads * G + hq] = S > 0.f ? (mx + fast_log2(S)) * kLn2 : -INFINITY;
 }
 
 template <int D>
@@ -1211,37 +1591,41 @@ std::vector<int64_t> cut_segments(const int32_t* indptr, int batch, int64_t tota
   return cut;
 }
 
-// KV heads per workgroup of the streaming kernel: 8 (one block-row slice of
-// 2 KB per token) for the head_dim-128 kernel when the heads divide evenly
-// and the register budget allows two waves per SIMD, else one; the register
-// kernel always groups 4 heads (and idles waves past the last head).
-int heads_per_workgroup(int group, int head_dim, int num_kv_heads) {
-  if (head_dim != 128) return 4;
-  return (group <= 4 && num_kv_heads % 8 == 0) ? 8 : 1;
+// Whether a head layout has the LDS kernel.
+bool lds_layout(int group, int head_dim, int num_kv_heads) {
+  return head_dim == 128 && group <= 4 && num_kv_heads % kLdsHeads == 0;
 }
 
-// Workgroups of the streaming kernel one CU holds at once (LDS- or
-// register-limited; from the compiled kernels' resources), used to size the
-// schedule.
-int resident_workgroups_per_cu(int group, int head_dim, int hpw) {
-  if (head_dim == 128) return hpw == 8 ? 1 : (group == 8 ? 4 : 8);
-  return group <= 2 ? 2 : 1;
+// KV heads per workgroup of the wave kernel: its waves are split between heads
+// and pages.  More heads read longer runs of each token row, fewer leave longer
+// segments and so fewer pieces to merge.
+int wave_heads(int head_dim, int num_kv_heads) {
+  if (num_kv_heads % 4 == 0) return 4;
+  return num_kv_heads == 2 || (head_dim != 128 && num_kv_heads % 2 == 0) ? 2 : 1;
+}
+
+// Whether a kernel takes a schedule's KV heads per workgroup.
+bool valid_heads_per_group(int group, int head_dim, int num_kv_heads, int hpw) {
+  if (hpw == kLdsHeads) return lds_layout(group, head_dim, num_kv_heads);
+  return (hpw == 1 || hpw == 2 || hpw == 4) && num_kv_heads % hpw == 0;
 }
 
 template <int G, int D>
 void launch_segments(const DecodeArgs& a, int segments, int head_groups, int hpw,
                      hipStream_t s) {
   const dim3 grid{unsigned(segments), unsigned(head_groups)};
-  if constexpr (D == 128) {
-    if constexpr (G <= 4) {
-      if (hpw == 8) {
-        decode_lds_kernel<G, 8><<<grid, 64 * 8, 0, s>>>(a);
-        return;
-      }
+  if constexpr (D == 128 && G <= 4) {
+    if (hpw == kLdsHeads) {
+      decode_lds_kernel<G><<<grid, 64 * kLdsHeads, 0, s>>>(a);
+      return;
     }
-    decode_lds_kernel<G, 1><<<grid, 64, 0, s>>>(a);
+  }
+  if constexpr (D == 256 && G == 8) {
+    DecodeArgs b = a;
+    b.q_splits = 2;
+    decode_wave_kernel<4, D><<<dim3{grid.x, 2 * grid.y}, 64 * WaveCfg<4, D>::kWaves, 0, s>>>(b);
   } else {
-    decode_reg_kernel<G, D><<<grid, kThreads, 0, s>>>(a);
+    decode_wave_kernel<G, D><<<grid, 64 * WaveCfg<G, D>::kWaves, 0, s>>>(a);
   }
 }
 
@@ -1337,29 +1721,34 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
     num_empty += indptr_host[b + 1] == indptr_host[b];
   }
   const int64_t total = batch > 0 ? indptr_host[batch] : 0;
-  const int hpw = heads_per_workgroup(group, head_dim, num_kv_heads);
-  const int head_groups = (num_kv_heads + hpw - 1) / hpw;
+  const bool lds = lds_layout(group, head_dim, num_kv_heads);
+  int hpw = lds ? kLdsHeads : wave_heads(head_dim, num_kv_heads);
+  // Workgroups a KV head group's segments share the CUs with (head_dim 256
+  // serves a group of 8 as two).
+  const int q_splits = head_dim == 256 && group == 8 ? 2 : 1;
 
-  // Segments per KV-head group: one resident workgroup each, at most
+  // Segments per KV-head group: one workgroup per CU, at most
   // kMaxSegPages pages each, at least one page each.  When the page cap
-  // forces more segments than there are resident slots, the count is rounded
+  // forces more segments than there are slots, the count is rounded
   // up to whole rounds of slots, so no round runs a few stragglers alone.
-  int64_t segs = 0;
-  if (total > 0) {
+  const int64_t slots = num_cus > 0 ? num_cus : 256;
+  auto segment_count = [&](int heads) -> int64_t {
+    if (total == 0) return 0;
     const int64_t at_least = (total + kMaxSegPages - 1) / kMaxSegPages;
+    int64_t n;
     if (num_segments_hint > 0) {
-      segs = std::max<int64_t>(num_segments_hint, at_least);
+      n = std::max<int64_t>(num_segments_hint, at_least);
     } else {
-      const int64_t slots = int64_t(num_cus > 0 ? num_cus : 256) *
-                            resident_workgroups_per_cu(group, head_dim, hpw);
-      const int64_t per_round = (slots + head_groups - 1) / head_groups;
-      segs = (std::max(per_round, at_least) + per_round - 1) / per_round * per_round;
+      const int64_t groups = int64_t(num_kv_heads / heads) * q_splits;
+      const int64_t per_round = (slots + groups - 1) / groups;
+      n = (std::max(per_round, at_least) + per_round - 1) / per_round * per_round;
     }
-    segs = std::min<int64_t>(segs, total);
-  }
+    return std::min<int64_t>(n, total);
+  };
+  int64_t segs = segment_count(hpw);
   KVC_REQUIRE(segs <= (int64_t(1) << 30), KVC_ERR_INVALID_ARG, "too many segments");
 
-  const std::vector<int64_t> cut = cut_segments(indptr_host, batch, total, segs);
+  std::vector<int64_t> cut = cut_segments(indptr_host, batch, total, segs);
 
   // Small batches (head_dim 128, no forced segment count): when every request
   // fits in kSmallMaxPages pages and the segments would cut a request,
@@ -1368,7 +1757,9 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
   int64_t max_pages = 0;
   for (int b = 0; b < batch; ++b)
     max_pages = std::max<int64_t>(max_pages, indptr_host[b + 1] - indptr_host[b]);
-  bool splits = false;
+  // (Where the wave kernel would stream the batch, a request of two pages or
+  // more is taken as cut: per-request workgroups are also its best schedule.)
+  bool splits = !lds && max_pages > 1;
   for (int64_t s = 1, bb = 0; s < segs && !splits; ++s) {
     const int64_t g = cut[size_t(s)];  // first page of segment s
     while (bb < batch && indptr_host[bb + 1] <= g) ++bb;
@@ -1421,6 +1812,39 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
     sched->append_pieces = 1;
     return ok();
   }
+
+  // Short requests without the per-request kernel (head_dim 64 / 256): one
+  // segment each, so that none is cut and no merge follows.
+  if (head_dim != 128 && num_segments_hint <= 0 && max_pages > 1 &&
+      max_pages <= kSmallMaxPages) {
+    cut.clear();
+    for (int i = 0; i < batch; ++i)
+      if (indptr_host[i + 1] > indptr_host[i]) cut.push_back(indptr_host[i]);
+    segs = int64_t(cut.size());
+    cut.push_back(total);
+  }
+
+  // Few pages for the LDS kernel's 8-head workgroups: at two or three pages
+  // each they are all start-up and cut a long request into up to 256 pieces.
+  // The wave kernel on 1, 2 or 4 heads per workgroup streams longer segments;
+  // the shorter the requests, the more heads, so that a workgroup's waves do
+  // not meet at a piece's end too often.  Measured with 8 KV heads, one layer
+  // with its append, LDS kernel -> 1 / 2 / 4 heads, in us:
+  //   group 4, requests x pages:  1 x 256  25.3 -> 12.9 / 13.8 / 17.8
+  //     8 x 68  18.3 -> 15.0 / 15.5 / 16.7     16 x 110  30.9 -> 30.3 / 28.9 / 28.3
+  //     20 x 37 19.9 -> 19.2 / 18.6 / 18.6     60 x 27   28.8 -> 30.2 / 27.9 / 27.6
+  //     12 x 14 12.5 -> 13.2 / 12.5 / 12.4     32 x 128  51.1 -> 55.0 / 51.7 / 50.7
+  //   groups 1, 2 (the LDS kernel's arithmetic is a quarter or half of that):
+  //     2 x 138 18.3 -> 13.3 / 12.9 / 14.9     4 x 131   16.6 -> 16.4 / 15.5 / 16.0
+  //     8 x 72  14.7 -> 16.2 / 15.4 / 14.8     20 x 37   16.6 -> 19.2 / 17.9 / 17.4
+  const int64_t work = total * (num_kv_heads / kLdsHeads);  // pages of 8 heads
+  const int64_t mean = total / std::max(1, batch - num_empty);  // pages per request
+  if (lds && num_segments_hint <= 0 && work <= 12 * slots && mean >= (group == 4 ? 16 : 96)) {
+    hpw = group < 4 ? 2 : mean < 48 ? 4 : work <= 3 * slots ? 1 : 2;
+    segs = segment_count(hpw);
+    cut = cut_segments(indptr_host, batch, total, segs);
+  }
+  const int head_groups = num_kv_heads / hpw;
 
   const int64_t need = kvc_decode_plan_ints(batch, int32_t(segs));
   sched->batch = batch;
@@ -1517,9 +1941,8 @@ int decode_run(const kvc_decode_schedule* sched, const int32_t* plan, const void
                   (small ? (D == 128 && sched->heads_per_group == 1 &&
                             sched->num_head_groups == Hkv && sched->num_segments == batch &&
                             sched->num_pieces == batch && sched->max_partitions == 1)
-                         : (sched->heads_per_group == heads_per_workgroup(group, D, Hkv) &&
-                            sched->num_head_groups ==
-                                (Hkv + sched->heads_per_group - 1) / sched->heads_per_group)) &&
+                         : (valid_heads_per_group(group, D, Hkv, sched->heads_per_group) &&
+                            sched->num_head_groups == Hkv / sched->heads_per_group)) &&
                   sched->plan_ints == kvc_decode_plan_ints(batch, sched->num_segments),
               KVC_ERR_INVALID_ARG, "schedule not produced by kvc_decode_plan");
   KVC_REQUIRE(num_blocks > 0 && num_indices >= sched->total_pages, KVC_ERR_INVALID_ARG,
@@ -1580,20 +2003,22 @@ int decode_run(const kvc_decode_schedule* sched, const int32_t* plan, const void
   a.new_v = static_cast<const uint16_t*>(new_value);
   a.new_k_stride = new_key_stride;
   a.new_v_stride = new_value_stride;
+  a.heads_per_group = sched->heads_per_group;
+  a.q_splits = 1;
   if (new_key || new_value) {
     KVC_REQUIRE(new_key && new_value, KVC_ERR_INVALID_ARG, "new_key and new_value go together");
-    KVC_REQUIRE(D == 128 &&
-                    (small || (sched->heads_per_group == 8 && sched->append_pieces <= kNewMax)),
-                KVC_ERR_UNSUPPORTED,
-                "fused append needs head_dim 128 and either a small-batch schedule or a "
-                "multiple of 8 KV heads with group <= 4 and at most " +
+    const bool lds = !small && sched->heads_per_group == kLdsHeads;
+    KVC_REQUIRE(!lds || sched->append_pieces <= kNewMax, KVC_ERR_UNSUPPORTED,
+                "with 8 KV heads per workgroup the append takes at most " +
                     std::to_string(kNewMax) + " leading pieces per segment holding request "
                     "ends (schedule->append_pieces)");
     KVC_REQUIRE(new_key_stride >= int64_t(Hkv) * D && new_value_stride >= int64_t(Hkv) * D,
                 KVC_ERR_INVALID_ARG, "new row stride smaller than a row");
-    KVC_REQUIRE(aligned(new_key, 16) && aligned(new_value, 16) && new_key_stride % 8 == 0 &&
-                    new_value_stride % 8 == 0,
-                KVC_ERR_ALIGNMENT, "new rows must be 16-byte aligned");
+    // The wave kernel takes any 4-byte aligned rows, the others 16-byte ones.
+    const int row_bytes = small || lds ? 16 : 4;
+    KVC_REQUIRE(aligned(new_key, row_bytes) && aligned(new_value, row_bytes) &&
+                    (new_key_stride * 2) % row_bytes == 0 && (new_value_stride * 2) % row_bytes == 0,
+                KVC_ERR_ALIGNMENT, "new rows must be " + std::to_string(row_bytes) + "-byte aligned");
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
 
@@ -1734,6 +2159,39 @@ extern "C" int kvc_batch_decode_run_noalloc(
 }
 
 extern "C" int kvc_batch_decode_append_run(
+    const kvc_decode_schedule* sched, const int32_t* plan, const void* q,
+    int64_t q_batch_stride, void* key_cache, void* value_cache,
+    int64_t cache_block_stride, int64_t cache_token_stride, int64_t num_blocks,
+    const int32_t* indptr, const int32_t* indices, int64_t num_indices,
+    const int32_t* last_page_len, const void* new_key, int64_t new_key_stride,
+    const void* new_value, int64_t new_value_stride, float sm_scale, void* workspace,
+    int64_t workspace_bytes, void* out, int64_t out_batch_stride, float* lse,
+    void* stream) {
+  KVC_REQUIRE(new_key && new_value, KVC_ERR_INVALID_ARG, "null new_key or new_value");
+  KVC_REQUIRE(sched, KVC_ERR_INVALID_ARG, "null schedule");
+  if (sched->batch > 0) {
+    const bool small = sched->small_batch != 0;
+    KVC_REQUIRE(sched->num_kv_heads > 0 && sched->head_dim == 128 &&
+                    (small || (lds_layout(sched->num_qo_heads / sched->num_kv_heads, 128,
+                                          sched->num_kv_heads) &&
+                               (sched->heads_per_group != kLdsHeads ||
+                                sched->append_pieces <= kNewMax))),
+                KVC_ERR_UNSUPPORTED,
+                "fused append needs head_dim 128 and either a small-batch schedule or a "
+                "multiple of 8 KV heads with group <= 4 and at most " +
+                    std::to_string(kNewMax) + " leading pieces per segment holding request "
+                    "ends (schedule->append_pieces)");
+    KVC_REQUIRE(aligned(new_key, 16) && aligned(new_value, 16) && new_key_stride % 8 == 0 &&
+                    new_value_stride % 8 == 0,
+                KVC_ERR_ALIGNMENT, "new rows must be 16-byte aligned");
+  }
+  return decode_run(sched, plan, q, q_batch_stride, key_cache, value_cache, cache_block_stride,
+                    cache_token_stride, num_blocks, indptr, indices, num_indices, last_page_len,
+                    new_key, new_key_stride, new_value, new_value_stride, sm_scale, workspace,
+                    workspace_bytes, out, out_batch_stride, lse, stream);
+}
+
+extern "C" int kvc_batch_decode_step_run(
     const kvc_decode_schedule* sched, const int32_t* plan, const void* q,
     int64_t q_batch_stride, void* key_cache, void* value_cache,
     int64_t cache_block_stride, int64_t cache_token_stride, int64_t num_blocks,

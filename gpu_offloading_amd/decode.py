@@ -77,7 +77,8 @@ class BatchDecodeWithPagedKVCacheWrapper:
         # (id(k), id(v)) -> (k ref, v ref, (ps, hkv, d), launch arguments)
         # for the cache tensors already checked (one pair per layer).
         self._kv_checked: dict = {}
-        self._fused_ok = False
+        self._fused_ok = False   # run_with_append is supported
+        self._appends = False    # some entry point appends in the decode launch
         self._cap_cache: dict = {}   # batch -> plan-image capacity
         ws = float_workspace_buffer
         self._ws_args = (ws.data_ptr(), ws.numel() * ws.element_size())
@@ -206,9 +207,17 @@ class BatchDecodeWithPagedKVCacheWrapper:
             self._meta_refs = (indptr_dev, indices_dev, lpl_dev)
             self._meta_args = (indptr_dev.data_ptr(), indices_dev.data_ptr(),
                                self._num_indices, lpl_dev.data_ptr())
-        self._fused_ok = (sched.head_dim == 128 and
+        # heads_per_group 8 is the kernel that stages pages in LDS; its append
+        # takes few request ends per segment.  The other kernels append whatever
+        # the schedule; run_with_append is offered for the layouts of the first.
+        staged = sched.small_batch == 0 and sched.heads_per_group == 8
+        hkv = sched.num_kv_heads
+        self._appends = not staged or sched.append_pieces <= 4
+        self._fused_ok = (sched.head_dim == 128 and self._appends and
                           (sched.small_batch == 1 or
-                           (sched.heads_per_group == 8 and sched.append_pieces <= 4)))
+                           (hkv % 8 == 0 and sched.num_qo_heads <= 4 * hkv)))
+        self._append_entry = ("kvc_batch_decode_append_run" if self._fused_ok
+                              else "kvc_batch_decode_step_run")
 
     # ------------------------------------------------- in-package fast path
     def _plan_capacity(self, batch: int) -> int:
@@ -284,8 +293,8 @@ class BatchDecodeWithPagedKVCacheWrapper:
     @property
     def fused_append_supported(self) -> bool:
         """Whether ``run_with_append`` can serve the planned batch (head_dim
-        128 and either a small-batch schedule or 8 KV heads per workgroup
-        with few request ends per segment)."""
+        128 and either a small-batch schedule or a multiple of 8 KV heads with
+        group <= 4 and few request ends per segment)."""
         return self._sched is not None and self._fused_ok
 
     def run_with_append(self, q: torch.Tensor,
@@ -304,13 +313,15 @@ class BatchDecodeWithPagedKVCacheWrapper:
         return self._launch(q, paged_kv_cache, out, lse, return_lse, sh, new_key, new_value)
 
     def _launch(self, q, paged_kv_cache, out, lse, return_lse, sh, new_key, new_value,
-                kv=None):
+                kv=None, any_layout=False):
         """Check the call's tensors against the plan and launch the decode
         (with the fused append when ``new_key`` is given) on stream ``sh``.
         The plan's and the cache's arguments were checked and converted once
         (``_adopt``, ``_kv_args``); per call only q, out, lse and the new rows
         are checked.  ``kv``: the cache's launch arguments, already checked
-        (``PagedKVCache`` passes those of its own layers)."""
+        (``PagedKVCache`` passes those of its own layers).  ``any_layout``:
+        append for every schedule with ``_appends``, not only those
+        ``run_with_append`` takes."""
         if self._sched is None:
             _fail("run() called before plan()")
         if kv is None:
@@ -344,7 +355,7 @@ class BatchDecodeWithPagedKVCacheWrapper:
                       *self._meta_args, self._sm_scale, *self._ws_args, out.data_ptr(),
                       out.stride(0), lse_p, sh)
             return (out, lse) if return_lse else out
-        if not self._fused_ok:
+        if not (self._fused_ok or any_layout):
             _fail("the fused append needs head_dim 128, num_kv_heads a multiple of 8, "
                   "group <= 4 and at most 4 request ends in a segment's leading pieces")
         for name, t in (("new_key", new_key), ("new_value", new_value)):
@@ -354,7 +365,7 @@ class BatchDecodeWithPagedKVCacheWrapper:
                 _fail(f"{name} must be bfloat16 [B, {hkv}, {d}] with contiguous heads")
             if t.get_device() != dev:
                 _fail(f"{name} on a different device than the workspace")
-        _lib.call("kvc_batch_decode_append_run", *self._pre_args, q.data_ptr(), qt[0], *kv,
+        _lib.call(self._append_entry, *self._pre_args, q.data_ptr(), qt[0], *kv,
                   *self._meta_args, new_key.data_ptr(), new_key.stride(0), new_value.data_ptr(),
                   new_value.stride(0), self._sm_scale, *self._ws_args, out.data_ptr(),
                   out.stride(0), lse_p, sh)

@@ -829,12 +829,18 @@ class PagedKVCache:
         ops.reshape_and_cache_flash(key, value, self.k_cache[layer], self.v_cache[layer],
                                     slot_mapping, "auto")
 
+    @staticmethod
+    def _word_rows(t: torch.Tensor) -> bool:
+        """Whether a step's new rows are 4-byte aligned (the decode launch
+        appends those; ``append`` takes any)."""
+        return (t.data_ptr() | (2 * t.stride(0))) % 4 == 0 if t.dim() == 3 else False
+
     def append_and_decode(self, layer: int, key: torch.Tensor, value: torch.Tensor,
                           q: torch.Tensor, out: Optional[torch.Tensor] = None,
                           return_lse: bool = False):
         """``append(layer, key, value, slots)`` then ``decode(layer, q)`` for
-        the step set up by the last ``prepare_decode_step``: one launch when
-        the decode wrapper supports the fused append, else the two calls.
+        the step set up by the last ``prepare_decode_step``: one launch
+        where the step's decode kernel appends, else the two calls.
         ``key``/``value`` are the step's new rows ``[B, Hkv, D]`` in the order
         of that call's ``seq_ids``; the result is the same either way, bit for
         bit."""
@@ -845,8 +851,8 @@ class PagedKVCache:
         w = self._decode_wrapper
         sh = self._step_stream_for_call()
         kv = self._layer_kv[layer]
-        if w._fused_ok:
-            return w._launch(q, None, out, None, return_lse, sh, key, value, kv)
+        if w._fused_ok or (w._appends and self._word_rows(key) and self._word_rows(value)):
+            return w._launch(q, None, out, None, return_lse, sh, key, value, kv, True)
         self.append(layer, key, value, slots)
         return w._launch(q, None, out, None, return_lse, sh, None, None, kv)
 

@@ -131,7 +131,7 @@ typedef struct kvc_decode_schedule {
   int32_t head_dim;
   int32_t page_size;
   int32_t num_segments;     /* segments per group of KV heads              */
-  int32_t num_head_groups;  /* ceil(num_kv_heads / heads_per_group)        */
+  int32_t num_head_groups;  /* num_kv_heads / heads_per_group              */
   int32_t num_pieces;
   int32_t pieces_offset;    /* int32 offsets inside the plan image         */
   int32_t nparts_offset;
@@ -142,7 +142,8 @@ typedef struct kvc_decode_schedule {
   int64_t plan_ints;        /* int32 entries of the plan image             */
   int64_t workspace_bytes;  /* bytes kvc_batch_decode_run will use         */
   int32_t append_pieces;    /* most leading pieces of a segment that reach
-                               a request end (fused append supports <= 4)  */
+                               a request end (the fused append supports
+                               <= 4 where heads_per_group is 8)            */
   int32_t small_batch;      /* 1: one workgroup per (request, KV head), its
                                waves splitting the pages (see below)       */
 } kvc_decode_schedule;
@@ -212,10 +213,28 @@ int kvc_batch_decode_run_noalloc(
  * indices[indptr[b+1]-1], offset last_page_len[b]-1, i.e. the slot the step's
  * slot mapping gives it -- and attended with the rest of the request.
  * Requests with no pages append nothing.  The cache and the output equal
- * those of the two separate calls bit for bit.  Needs head_dim 128, a
- * multiple of 8 KV heads, group <= 4 and schedule->append_pieces <= 4;
- * otherwise KVC_ERR_UNSUPPORTED (the caller then makes the two calls). */
+ * those of the two separate calls bit for bit.  Needs head_dim 128 and either
+ * a small-batch schedule or a multiple of 8 KV heads, group <= 4 and, where
+ * heads_per_group is 8, append_pieces <= 4; otherwise KVC_ERR_UNSUPPORTED (the
+ * caller then makes the two calls, or calls kvc_batch_decode_step_run). */
 int kvc_batch_decode_append_run(
+    const kvc_decode_schedule* schedule, const int32_t* plan,
+    const void* q, int64_t q_batch_stride,
+    void* key_cache, void* value_cache,
+    int64_t cache_block_stride, int64_t cache_token_stride,
+    int64_t num_blocks, const int32_t* indptr, const int32_t* indices,
+    int64_t num_indices, const int32_t* last_page_len,
+    const void* new_key, int64_t new_key_stride,
+    const void* new_value, int64_t new_value_stride, float sm_scale,
+    void* workspace, int64_t workspace_bytes, void* out,
+    int64_t out_batch_stride, float* lse, void* stream);
+
+/* kvc_batch_decode_append_run for the other schedules too: any head_dim, group
+ * and number of KV heads that kvc_decode_plan accepts, same arguments, same
+ * result.  Refused with KVC_ERR_UNSUPPORTED only where a schedule has
+ * heads_per_group 8 and append_pieces > 4.  new_key / new_value rows 16-byte
+ * aligned for schedules with small_batch or heads_per_group 8, else 4-byte. */
+int kvc_batch_decode_step_run(
     const kvc_decode_schedule* schedule, const int32_t* plan,
     const void* q, int64_t q_batch_stride,
     void* key_cache, void* value_cache,
