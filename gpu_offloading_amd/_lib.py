@@ -74,6 +74,20 @@ class KvcPrefillSchedule(ctypes.Structure):
     ]
 
 
+class KvcPrefillSplit(ctypes.Structure):
+    """Mirror of ``kvc_prefill_split`` (include/kvc.h)."""
+
+    _fields_ = [
+        ("num_units", c_int32),
+        ("num_parts", c_int32),
+        ("num_merges", c_int32),
+        ("parts_offset", c_int32),
+        ("merges_offset", c_int32),
+        ("base_offset", c_int32),
+        ("workspace_bytes", c_int64),
+    ]
+
+
 class KvcDecodeStepLayout(ctypes.Structure):
     """Mirror of ``kvc_decode_step_layout`` (include/kvc.h)."""
 
@@ -133,6 +147,12 @@ SIGNATURES = {
     "kvc_prefill_plan": (c_int, [
         c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,
         POINTER(KvcPrefillSchedule), c_void_p, c_int64]),
+    "kvc_prefill_plan_split": (c_int, [
+        c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,
+        POINTER(KvcPrefillSchedule), POINTER(KvcPrefillSplit), c_void_p, c_int64]),
+    "kvc_batch_prefill_split_run": (c_int, [
+        POINTER(KvcPrefillSchedule), POINTER(KvcPrefillSplit), _I32P, _P, c_int64, _P, c_int64,
+        _P, _P, c_int64, c_int64, c_int64, _I32P, c_int64, c_float, _P, c_int64, _P, _P]),
     "kvc_batch_prefill_run": (c_int, [
         POINTER(KvcPrefillSchedule), _I32P, _P, c_int64, _P, _P, c_int64, c_int64, c_int64,
         _I32P, c_int64, c_float, _P, c_int64, _P, _P]),

@@ -97,6 +97,11 @@ struct PrefillArgs {
   uint16_t* out;
   int64_t out_stride;      // elements between output tokens
   float* lse;              // [total_q][Hq] natural log, may be null
+  // Split plans: unit u leaves its rows in partial unit_part[u] (-1: it writes
+  // the output), 256 rows of 128 fp32 values and 256 log2-sum-exps each.
+  const int32_t* unit_part;
+  float* part_o;
+  float* part_lse;
 };
 
 // K rows of 256 B whose 16-byte chunks are XOR-swizzled by key: chunk c of
@@ -154,7 +159,10 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 // offset, key tiles, pages) of one query tile of one request.
 struct Unit { int h, tok0, q_len, kv_len, q_off, page_off, ntiles, npages; };
 
-template <int G>
+// kSplit: units may cover part of a tile's keys.  Such a unit's record has its
+// lengths and page offset moved to its first key, so everything up to the end
+// of the unit is the same; the bulk kernel is built without the difference.
+template <int G, bool kSplit>
 __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(PrefillArgs a) {
   constexpr int kTokPerWave = kWaveRows / G;
   // One LDS object, so that the K/V tiles sit in its first 64 KB (operand
@@ -501,59 +509,77 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(PrefillArgs a
   // The stores are non-temporal: the output is not read again here, and
   // leaving it out of the caches keeps the K/V tiles the other query tiles
   // of a request re-read there.
-  auto finish_unit = [&]() __attribute__((always_inline)) {
+  auto finish_unit = [&](int k) __attribute__((always_inline)) {
     const float l_run = l_half + __shfl_xor(l_half, 32);
     const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-    uint8_t* stg = lds.ostage[wave];
-    // O^T column r = this row; entry (db, 4i+j) = head dim 32db + 8i + 4half + j,
-    // so (db, i) is the row's 16-byte chunk 4db + i and half its 8-byte half.
-    uint8_t* wr = stg + r * kORow + 8 * half;
+    const int part = kSplit ? __builtin_amdgcn_readfirstlane(a.unit_part[u_first + k]) : -1;
+    if (kSplit && part >= 0) {
+      // A piece of the tile's keys: the rows in fp32, merged by a later kernel.
+      if (row_ok) {
+        const int64_t row = int64_t(part) * kTileRows + wave * kWaveRows + r;
+        float* po = a.part_o + row * kD + 4 * half;
 #pragma unroll
-    for (int db = 0; db < 4; ++db) {
+        for (int db = 0; db < 4; ++db)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<uint2*>(wr + 16 * (4 * db + i)) =
-            make_uint2(pack_bf16(o[db][4 * i] * inv, o[db][4 * i + 1] * inv),
-                       pack_bf16(o[db][4 * i + 2] * inv, o[db][4 * i + 3] * inv));
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // Row 4t + q (q = L/16 < 4) is token (4t + q) / G of the wave, head
-    // (4t + q) % G: for G <= 4 that is token t (4/G) + q/G, head q % G; for
-    // G >= 4 token 4t/G, head 4t % G + q.  So the lane's part of the address
-    // is set once and the store's part is uniform.
-    const int c = lane & 15;
-    const int q = lane >> 4;
-    const int wave_tok = cu.tok0 + wave * kTokPerWave;
-    const int toks_left = cu.q_len - wave_tok;
-    const int lane_tok = G <= 4 ? q / G : 0;
-    const int lane_head = G <= 4 ? q % G : q;
-    uint16_t* obase = a.out + int64_t(cu.q_off + wave_tok + lane_tok) * a.out_stride +
-                      int64_t(cu.h * G + lane_head) * kD + 8 * c;
-    const uint8_t* rd = stg + q * kORow + 16 * c;
-    // Four read-backs in flight, then their four stores (one at a time, each
-    // store waited for its own read).
-#pragma unroll
-    for (int t0 = 0; t0 < kWaveRows / 4; t0 += 4) {
-      uint4 v[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        v[i] = *reinterpret_cast<const uint4*>(rd + 4 * (t0 + i) * kORow);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int t = t0 + i;
-        const int t_tok = G <= 4 ? t * (4 / G) : 4 * t / G;
-        const int t_head = G <= 4 ? 0 : 4 * t % G;
-        if (t_tok + lane_tok < toks_left)
-          store_stream(obase + int64_t(t_tok) * a.out_stride + t_head * kD, v[i]);
+          for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<float4*>(po + 32 * db + 8 * i) =
+                make_float4(o[db][4 * i] * inv, o[db][4 * i + 1] * inv, o[db][4 * i + 2] * inv,
+                            o[db][4 * i + 3] * inv);
+        // (l_run NaN stays NaN, l_run 0 gives -inf)
+        if (half == 0) a.part_lse[row] = l_run == 0.f ? -INFINITY : m_run + fast_log2(l_run);
       }
-      __builtin_amdgcn_sched_barrier(0);
+    } else {
+      uint8_t* stg = lds.ostage[wave];
+      // O^T column r = this row; entry (db, 4i+j) = head dim 32db + 8i + 4half + j,
+      // so (db, i) is the row's 16-byte chunk 4db + i and half its 8-byte half.
+      uint8_t* wr = stg + r * kORow + 8 * half;
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          *reinterpret_cast<uint2*>(wr + 16 * (4 * db + i)) =
+              make_uint2(pack_bf16(o[db][4 * i] * inv, o[db][4 * i + 1] * inv),
+                         pack_bf16(o[db][4 * i + 2] * inv, o[db][4 * i + 3] * inv));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      // Row 4t + q (q = L/16 < 4) is token (4t + q) / G of the wave, head
+      // (4t + q) % G: for G <= 4 that is token t (4/G) + q/G, head q % G; for
+      // G >= 4 token 4t/G, head 4t % G + q.  So the lane's part of the address
+      // is set once and the store's part is uniform.
+      const int c = lane & 15;
+      const int q = lane >> 4;
+      const int wave_tok = cu.tok0 + wave * kTokPerWave;
+      const int toks_left = cu.q_len - wave_tok;
+      const int lane_tok = G <= 4 ? q / G : 0;
+      const int lane_head = G <= 4 ? q % G : q;
+      uint16_t* obase = a.out + int64_t(cu.q_off + wave_tok + lane_tok) * a.out_stride +
+                        int64_t(cu.h * G + lane_head) * kD + 8 * c;
+      const uint8_t* rd = stg + q * kORow + 16 * c;
+      // Four read-backs in flight, then their four stores (one at a time, each
+      // store waited for its own read).
+#pragma unroll
+      for (int t0 = 0; t0 < kWaveRows / 4; t0 += 4) {
+        uint4 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          v[i] = *reinterpret_cast<const uint4*>(rd + 4 * (t0 + i) * kORow);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int t = t0 + i;
+          const int t_tok = G <= 4 ? t * (4 / G) : 4 * t / G;
+          const int t_head = G <= 4 ? 0 : 4 * t % G;
+          if (t_tok + lane_tok < toks_left)
+            store_stream(obase + int64_t(t_tok) * a.out_stride + t_head * kD, v[i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (row_ok && a.lse && half == 0)
+        a.lse[int64_t(cu.q_off + tok) * Hq + hq] =
+            l_run > 0.f ? (m_run + fast_log2(l_run)) * kLn2 : -INFINITY;
     }
-    if (row_ok && a.lse && half == 0)
-      a.lse[int64_t(cu.q_off + tok) * Hq + hq] =
-          l_run > 0.f ? (m_run + fast_log2(l_run)) * kLn2 : -INFINITY;
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
@@ -629,7 +655,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(PrefillArgs a
           if (has_next) load_q(nu, qb);
           mfma(n, yes{}, no{});
           __syncthreads();
-          finish_unit();
+          finish_unit(k);
           __syncthreads();
         } else {
           // Team 1 stages K_{j+1} and V_j at the start of slot 2j, from
@@ -687,12 +713,12 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(PrefillArgs a
           mfma(n, yes{}, no{});
           wait_dma();
           __syncthreads();
-          finish_unit();
+          finish_unit(k);
         }
       } else {
         prefetch_next(k);
         if (has_next) load_q(nu, qb);
-        finish_unit();
+        finish_unit(k);
       }
       if (has_next) {
         staged = n > 0 && nu.ntiles > 0;
@@ -707,9 +733,68 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(PrefillArgs a
   else run(std::integral_constant<int, 1>{});
 }
 
+// Merge of the split tiles: workgroup (tile x KV head, 16 of its 256 rows); 16
+// threads per row fold its partials, eight dims each, with the log-sum-exp rule.
+// Bound by latency: a few partials per row, read four at a time, all from L2 or
+// MALL where the pieces just left them.
+// Record: (KV head, first output token, rows, first partial, partials, 0, 0, 0).
 template <int G>
-void launch(const PrefillArgs& a, int workgroups, hipStream_t s) {
-  prefill_mfma_kernel<G><<<dim3(unsigned(workgroups)), kThreads, 0, s>>>(a);
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, const int4* merges) {
+  const int4 rec = merges[2 * blockIdx.x];
+  const int nparts = merges[2 * blockIdx.x + 1].x;
+  const int row = blockIdx.y * 16 + (threadIdx.x >> 4);
+  const int c = threadIdx.x & 15;
+  if (row >= rec.z) return;
+  const int64_t p0 = int64_t(rec.w) * kTileRows + row;
+  float mx = -INFINITY;
+  for (int p = 0; p < nparts; ++p) mx = fmaxf(mx, a.part_lse[p0 + int64_t(p) * kTileRows]);
+  if (mx == -INFINITY) mx = 0.f;  // no key in any: weights 0 (and NaN where a partial is NaN)
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, S = 0.f;
+  constexpr int kAhead = 4;  // partials in flight per thread
+  for (int q0 = 0; q0 < nparts; q0 += kAhead) {
+    float4 x[kAhead][2];
+    float w[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int64_t pr = p0 + int64_t(min(q0 + i, nparts - 1)) * kTileRows;
+      const float4* src = reinterpret_cast<const float4*>(a.part_o + pr * kD + 8 * c);
+      x[i][0] = src[0];
+      x[i][1] = src[1];
+      w[i] = fast_exp2(a.part_lse[pr] - mx);
+    }
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      if (q0 + i < nparts) {
+        S += w[i];
+        const float v[8] = {x[i][0].x, x[i][0].y, x[i][0].z, x[i][0].w,
+                            x[i][1].x, x[i][1].y, x[i][1].z, x[i][1].w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = fmaf(w[i], v[e], acc[e]);
+      }
+    }
+  }
+  const float inv = S > 0.f ? 1.f / S : 0.f;
+  const int64_t tok = rec.y + row / G;
+  const int hq = rec.x * G + row % G;
+  uint32_t w[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) w[e] = pack_bf16(acc[2 * e] * inv, acc[2 * e + 1] * inv);
+  *reinterpret_cast<uint4*>(a.out + tok * a.out_stride + int64_t(hq) * kD + 8 * c) =
+      make_uint4(w[0], w[1], w[2], w[3]);
+  if (a.lse && c == 0)
+    a.lse[tok * a.num_kv_heads * G + hq] =
+        S > 0.f ? (mx + fast_log2(S)) * kLn2 : -INFINITY;
+}
+
+template <int G>
+void launch(const PrefillArgs& a, int workgroups, const int4* merges, int num_merges,
+            hipStream_t s) {
+  if (!a.unit_part) {
+    prefill_mfma_kernel<G, false><<<dim3(unsigned(workgroups)), kThreads, 0, s>>>(a);
+    return;
+  }
+  prefill_mfma_kernel<G, true><<<dim3(unsigned(workgroups)), kThreads, 0, s>>>(a);
+  prefill_merge_kernel<G><<<dim3(unsigned(num_merges), kTileRows / 16), 256, 0, s>>>(a, merges);
 }
 
 // Persistent workgroups: at most one per CU of an MI355X (256), each running
@@ -722,17 +807,245 @@ int64_t plan_ints_for(int64_t items, int hkv) {
   return plan_table_ints(plan_workgroups(items, hkv)) + items * hkv * kItemInts;
 }
 
-}  // namespace
-}  // namespace kvc
+// Split plans.  A batch of few query tiles over long histories has fewer units
+// than the chip has CUs, or a few long ones: 3 chunks of 60-400 tokens over
+// 3000-8000 tokens (8 KV heads, group 4) are 80 units of about 100 key tiles,
+// 157 us with 176 CUs idle.  Units are then cut into pieces of about `piece`
+// key tiles, which leave fp32 partials that a second kernel merges: 90 us; 3
+// chunks of 40 tokens over 25000-29000 tokens of one head 546 -> 54 us.  A unit
+// costs its key tiles + kUnitCost (its start and end, 4.6-6.4 us against 1.6 us
+// per tile) and the second launch kMergeCost; the plan takes the pieces that
+// end soonest by that, and whole units if none is a tenth sooner.  Units of up
+// to kSplitTiles tiles stay whole (the merge costs what cutting them gives), and
+// so do batches of more than kSplitMaxUnits units, which fill the chip.
+constexpr int kSplitTiles = 16;
+constexpr int kMinPiece = 4;       // tiles; shorter ones are mostly start and end
+constexpr int kUnitCost = 4;
+constexpr int kMergeCost = 5;       // the merge launch, in tiles
+constexpr int64_t kSplitMaxUnits = 512;
+constexpr int64_t kMaxPieces = 768;  // units of a split plan: at most 101 MB of partials
 
-using namespace kvc;
+// End of the longest workgroup when units of these costs are dealt longest
+// first to the least loaded of W workgroups.
+int64_t makespan(std::vector<int>& costs, int64_t W) {
+  std::sort(costs.begin(), costs.end(), std::greater<int>());
+  std::priority_queue<int64_t, std::vector<int64_t>, std::greater<int64_t>> q;
+  for (int64_t i = 0; i < W; ++i) q.push(0);
+  int64_t end = 0;
+  for (const int c : costs) {
+    const int64_t t = q.top() + c;
+    q.pop();
+    q.push(t);
+    end = std::max(end, t);
+  }
+  return end;
+}
 
-extern "C" int kvc_prefill_plan(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host,
-                                const int32_t* last_page_len_host, int32_t batch,
-                                int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim,
-                                int32_t page_size, int32_t causal,
-                                kvc_prefill_schedule* sched, int32_t* plan_host,
-                                int64_t plan_capacity) {
+int pieces_of(int tiles, int piece) {
+  return tiles > kSplitTiles ? (tiles + piece - 1) / piece : 1;
+}
+
+// Key tiles per piece that end a batch of these units soonest, or 0 to leave
+// them whole (unless splitting saves a tenth).
+int split_piece(const std::vector<int32_t>& rec, int64_t n, int hkv) {
+  if (n * hkv > kSplitMaxUnits) return 0;
+  int64_t total = 0;
+  int longest = 0;
+  std::vector<int> costs;
+  for (int64_t i = 0; i < n; ++i) {
+    const int t = rec[i * kItemInts + 6];
+    total += int64_t(t) * hkv;
+    longest = std::max(longest, t);
+    costs.insert(costs.end(), size_t(hkv), t + kUnitCost);
+  }
+  if (longest <= kSplitTiles) return 0;
+  const int64_t share = (total + n * hkv * kUnitCost) / kMaxWorkgroups;
+  const int64_t whole = makespan(costs, kMaxWorkgroups);
+  if (whole <= share + share / 8) return 0;
+  int best = 0;
+  int64_t best_end = whole - whole / 10;
+  int last = 0;
+  // Pieces of two workgroups' shares of all tiles, of one, of two thirds of one
+  // and of half of one.
+  for (int k = 1; k <= 4; ++k) {
+    const int piece = int(std::max<int64_t>(kMinPiece, (2 * total + k * kMaxWorkgroups - 1) /
+                                                           (k * kMaxWorkgroups)));
+    if (piece == last || piece >= longest) continue;
+    last = piece;
+    costs.clear();
+    for (int64_t i = 0; i < n; ++i) {
+      const int t = rec[i * kItemInts + 6];
+      const int np = pieces_of(t, piece);
+      for (int x = 0; x < np; ++x)
+        costs.insert(costs.end(), size_t(hkv),
+                     int(int64_t(t) * (x + 1) / np - int64_t(t) * x / np) + kUnitCost);
+    }
+    if (int64_t(costs.size()) > kMaxPieces) continue;
+    const int64_t end = makespan(costs, kMaxWorkgroups) + kMergeCost;
+    if (end < best_end) {
+      best_end = end;
+      best = piece;
+    }
+  }
+  return best;
+}
+
+// int32 entries of a split plan's image: the workgroups' table, the unit
+// records, each unit's partial (padded to 4) and the merge records.
+int64_t split_plan_ints(int64_t units, int64_t merges) {
+  return plan_table_ints(std::min(kMaxWorkgroups, units)) + units * kItemInts +
+         (units + 3) / 4 * 4 + merges * kItemInts;
+}
+
+// The plan of whole units: plan_ints_for(n, hkv) entries.
+void write_plan(const std::vector<int32_t>& rec, int64_t n, int hkv, int32_t* plan_host) {
+  // Longest items first: the causal tail of short tiles fills the gaps.
+  std::vector<int64_t> order(n);
+  for (int64_t i = 0; i < n; ++i) order[i] = i;
+  std::stable_sort(order.begin(), order.end(), [&](int64_t x, int64_t y) {
+    return rec[x * kItemInts + 6] > rec[y * kItemInts + 6];
+  });
+  // Units (item, KV head) in the order a grid of (items, heads) workgroups
+  // would be dispatched: head-major, items longest first.  The hardware
+  // hands workgroup w to XCD w % 8 and each XCD's next workgroup to its
+  // first free CU; the plan replays that list scheduling with each unit's
+  // cost taken as its key tiles + 2, assigning unit d to a workgroup of XCD
+  // d % 8 (workgroup b runs on XCD b % 8), so the units of one request and
+  // head still run side by side on one XCD and share its L2.
+  const int64_t units = n * hkv;
+  const int64_t W = plan_workgroups(n, hkv);
+  const int groups = (W % 8 == 0) ? 8 : 1;
+  std::vector<std::vector<int64_t>> lists(W);
+  {
+    typedef std::pair<int64_t, int64_t> Slot;  // (load, workgroup)
+    std::vector<std::priority_queue<Slot, std::vector<Slot>, std::greater<Slot>>> free_at(groups);
+    for (int64_t b = 0; b < W; ++b) free_at[b % groups].push(Slot(0, b));
+    for (int64_t d = 0; d < units; ++d) {
+      auto& q = free_at[d % groups];
+      const Slot sl = q.top();
+      q.pop();
+      lists[sl.second].push_back(d);
+      const int64_t item = order[d % n];
+      q.push(Slot(sl.first + rec[item * kItemInts + 6] + 2, sl.second));
+    }
+  }
+  const int64_t table = plan_table_ints(W);
+  std::fill_n(plan_host, table, 0);
+  int64_t next = 0;
+  for (int64_t b = 0; b < W; ++b) {
+    plan_host[2 * b] = int32_t(next);
+    plan_host[2 * b + 1] = int32_t(lists[b].size());
+    for (const int64_t d : lists[b]) {
+      int32_t* dst = plan_host + table + next * kItemInts;
+      std::copy_n(rec.data() + order[d % n] * kItemInts, kItemInts, dst);
+      dst[0] = int32_t(d / n);  // the KV head
+      ++next;
+    }
+  }
+}
+
+int split_plan(const std::vector<int32_t>& rec, int64_t n, int hkv, int piece, int tile_tokens,
+               int group, kvc_prefill_schedule* sched, kvc_prefill_split* split,
+               int32_t* plan_host, int64_t plan_capacity) {
+  struct Piece {
+    int64_t item;
+    int first, tiles, index;   // key tiles; index within its tile's pieces
+  };
+  std::vector<Piece> pieces;   // of one KV head
+  std::vector<int> count(static_cast<size_t>(n));
+  int64_t split_items = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    const int t = rec[i * kItemInts + 6];
+    const int np = pieces_of(t, piece);
+    count[size_t(i)] = np;
+    split_items += np > 1;
+    for (int x = 0; x < np; ++x) {
+      const int t0 = int(int64_t(t) * x / np), t1 = int(int64_t(t) * (x + 1) / np);
+      pieces.push_back(Piece{i, t0, t1 - t0, x});
+    }
+  }
+  const int64_t per_head = int64_t(pieces.size()), units = per_head * hkv;
+  const int64_t merges = split_items * hkv, W = std::min(kMaxWorkgroups, units);
+  std::vector<int64_t> first(static_cast<size_t>(n), -1);  // partial of piece 0, per head 0
+  int64_t parts = 0;
+  for (int64_t i = 0; i < n; ++i)
+    if (count[size_t(i)] > 1) {
+      first[size_t(i)] = parts;
+      parts += count[size_t(i)];
+    }
+  const int64_t parts_per_head = parts;
+  parts *= hkv;
+  const int64_t table = plan_table_ints(W);
+  const int64_t base = split_plan_ints(units, merges);
+  sched->plan_ints = base + plan_ints_for(n, hkv);
+  split->num_units = int32_t(units);
+  split->num_parts = int32_t(parts);
+  split->num_merges = int32_t(merges);
+  split->parts_offset = int32_t(table + units * kItemInts);
+  split->merges_offset = int32_t(split->parts_offset + (units + 3) / 4 * 4);
+  split->base_offset = int32_t(base);
+  split->workspace_bytes = parts * kTileRows * (kD + 1) * 4;
+  KVC_REQUIRE(plan_host && plan_capacity >= sched->plan_ints, KVC_ERR_WORKSPACE,
+              "plan buffer too small: need " + std::to_string(sched->plan_ints) + " int32");
+  // Longest first, to the least loaded workgroup.
+  std::vector<int64_t> order(static_cast<size_t>(units));
+  for (int64_t u = 0; u < units; ++u) order[size_t(u)] = u;
+  auto key = [&](int64_t u) { return pieces[size_t(u % per_head)]; };
+  std::stable_sort(order.begin(), order.end(),
+                   [&](int64_t x, int64_t y) { return key(x).tiles > key(y).tiles; });
+  std::vector<std::vector<int64_t>> lists(static_cast<size_t>(W));
+  typedef std::pair<int64_t, int64_t> Slot;  // (load, workgroup)
+  std::priority_queue<Slot, std::vector<Slot>, std::greater<Slot>> free_at;
+  for (int64_t b = 0; b < W; ++b) free_at.push(Slot(0, b));
+  for (const int64_t u : order) {
+    const Slot sl = free_at.top();
+    free_at.pop();
+    lists[size_t(sl.second)].push_back(u);
+    free_at.push(Slot(sl.first + key(u).tiles + kUnitCost, sl.second));
+  }
+  std::fill_n(plan_host, table, 0);
+  int32_t* unit_part = plan_host + split->parts_offset;
+  std::fill(unit_part, plan_host + split->merges_offset, -1);
+  int64_t next = 0;
+  for (int64_t b = 0; b < W; ++b) {
+    plan_host[2 * b] = int32_t(next);
+    plan_host[2 * b + 1] = int32_t(lists[size_t(b)].size());
+    for (const int64_t u : lists[size_t(b)]) {
+      const Piece p = key(u);
+      const int64_t head = u / per_head;
+      int32_t* dst = plan_host + table + next * kItemInts;
+      std::copy_n(rec.data() + p.item * kItemInts, kItemInts, dst);
+      const int pages = std::min<int>(dst[7], p.first * (kKeys / kPage));
+      dst[0] = int32_t(head);
+      dst[3] -= p.first * kKeys;   // keys from the piece's first on
+      dst[5] += pages;
+      dst[6] = p.tiles;
+      dst[7] -= pages;
+      if (count[size_t(p.item)] > 1)
+        unit_part[next] = int32_t(head * parts_per_head + first[size_t(p.item)] + p.index);
+      ++next;
+    }
+  }
+  int32_t* m = plan_host + split->merges_offset;
+  for (int64_t head = 0; head < hkv; ++head)
+    for (int64_t i = 0; i < n; ++i) {
+      if (count[size_t(i)] <= 1) continue;
+      const int32_t* r = rec.data() + i * kItemInts;
+      const int32_t out[kItemInts] = {int32_t(head), r[4] + r[1],
+                                      std::min(tile_tokens, r[2] - r[1]) * group,
+                                      int32_t(head * parts_per_head + first[size_t(i)]),
+                                      count[size_t(i)], 0, 0, 0};
+      m = std::copy_n(out, kItemInts, m);
+    }
+  write_plan(rec, n, hkv, plan_host + base);
+  return ok();
+}
+
+int prefill_plan(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host,
+                 const int32_t* last_page_len_host, int32_t batch, int32_t num_qo_heads,
+                 int32_t num_kv_heads, int32_t head_dim, int32_t page_size, int32_t causal,
+                 kvc_prefill_schedule* sched, kvc_prefill_split* split, int32_t* plan_host,
+                 int64_t plan_capacity) {
   KVC_REQUIRE(sched, KVC_ERR_INVALID_ARG, "null schedule");
   KVC_REQUIRE(batch >= 0, KVC_ERR_INVALID_ARG, "negative batch");
   KVC_REQUIRE(batch == 0 || (qo_indptr_host && kv_indptr_host && last_page_len_host),
@@ -785,67 +1098,72 @@ extern "C" int kvc_prefill_plan(const int32_t* qo_indptr_host, const int32_t* kv
   sched->total_q = int32_t(std::min<int64_t>(total_q, INT32_MAX));
   sched->max_key_tiles = max_tiles;
   sched->plan_ints = plan_ints_for(n, num_kv_heads);
+  if (split) {
+    *split = kvc_prefill_split{};
+    split->num_units = int32_t(n * num_kv_heads);
+    const int piece = split_piece(rec, n, num_kv_heads);
+    if (piece > 0)
+      return split_plan(rec, n, num_kv_heads, piece, tile_tokens, group, sched, split, plan_host,
+                        plan_capacity);
+  }
   KVC_REQUIRE(plan_host && plan_capacity >= sched->plan_ints, KVC_ERR_WORKSPACE,
               "plan buffer too small: need " + std::to_string(sched->plan_ints) + " int32");
-  // Longest items first: the causal tail of short tiles fills the gaps.
-  std::vector<int64_t> order(n);
-  for (int64_t i = 0; i < n; ++i) order[i] = i;
-  std::stable_sort(order.begin(), order.end(), [&](int64_t x, int64_t y) {
-    return rec[x * kItemInts + 6] > rec[y * kItemInts + 6];
-  });
-  // Units (item, KV head) in the order a grid of (items, heads) workgroups
-  // would be dispatched: head-major, items longest first.  The hardware
-  // hands workgroup w to XCD w % 8 and each XCD's next workgroup to its
-  // first free CU; the plan replays that list scheduling with each unit's
-  // cost taken as its key tiles + 2, assigning unit d to a workgroup of XCD
-  // d % 8 (workgroup b runs on XCD b % 8), so the units of one request and
-  // head still run side by side on one XCD and share its L2.
-  const int64_t units = n * num_kv_heads;
-  const int64_t W = plan_workgroups(n, num_kv_heads);
-  const int groups = (W % 8 == 0) ? 8 : 1;
-  std::vector<std::vector<int64_t>> lists(W);
-  {
-    typedef std::pair<int64_t, int64_t> Slot;  // (load, workgroup)
-    std::vector<std::priority_queue<Slot, std::vector<Slot>, std::greater<Slot>>> free_at(groups);
-    for (int64_t b = 0; b < W; ++b) free_at[b % groups].push(Slot(0, b));
-    for (int64_t d = 0; d < units; ++d) {
-      auto& q = free_at[d % groups];
-      const Slot sl = q.top();
-      q.pop();
-      lists[sl.second].push_back(d);
-      const int64_t item = order[d % n];
-      q.push(Slot(sl.first + rec[item * kItemInts + 6] + 2, sl.second));
-    }
-  }
-  const int64_t table = plan_table_ints(W);
-  std::fill_n(plan_host, table, 0);
-  int64_t next = 0;
-  for (int64_t b = 0; b < W; ++b) {
-    plan_host[2 * b] = int32_t(next);
-    plan_host[2 * b + 1] = int32_t(lists[b].size());
-    for (const int64_t d : lists[b]) {
-      int32_t* dst = plan_host + table + next * kItemInts;
-      std::copy_n(rec.data() + order[d % n] * kItemInts, kItemInts, dst);
-      dst[0] = int32_t(d / n);  // the KV head
-      ++next;
-    }
-  }
+  write_plan(rec, n, num_kv_heads, plan_host);
   return ok();
 }
 
-extern "C" int kvc_batch_prefill_run(const kvc_prefill_schedule* sched, const int32_t* plan,
-                                     const void* q, int64_t q_token_stride,
-                                     const void* key_cache, const void* value_cache,
-                                     int64_t cache_block_stride, int64_t cache_token_stride,
-                                     int64_t num_blocks, const int32_t* indices,
-                                     int64_t num_indices, float sm_scale, void* out,
-                                     int64_t out_token_stride, float* lse, void* stream) {
+}  // namespace
+}  // namespace kvc
+
+using namespace kvc;
+
+extern "C" int kvc_prefill_plan(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host,
+                                const int32_t* last_page_len_host, int32_t batch,
+                                int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim,
+                                int32_t page_size, int32_t causal,
+                                kvc_prefill_schedule* sched, int32_t* plan_host,
+                                int64_t plan_capacity) {
+  return prefill_plan(qo_indptr_host, kv_indptr_host, last_page_len_host, batch, num_qo_heads,
+                      num_kv_heads, head_dim, page_size, causal, sched, nullptr, plan_host,
+                      plan_capacity);
+}
+
+extern "C" int kvc_prefill_plan_split(const int32_t* qo_indptr_host,
+                                      const int32_t* kv_indptr_host,
+                                      const int32_t* last_page_len_host, int32_t batch,
+                                      int32_t num_qo_heads, int32_t num_kv_heads,
+                                      int32_t head_dim, int32_t page_size, int32_t causal,
+                                      kvc_prefill_schedule* sched, kvc_prefill_split* split,
+                                      int32_t* plan_host, int64_t plan_capacity) {
+  KVC_REQUIRE(split, KVC_ERR_INVALID_ARG, "null split");
+  return prefill_plan(qo_indptr_host, kv_indptr_host, last_page_len_host, batch, num_qo_heads,
+                      num_kv_heads, head_dim, page_size, causal, sched, split, plan_host,
+                      plan_capacity);
+}
+
+namespace {
+int prefill_run(const kvc_prefill_schedule* sched, const kvc_prefill_split* split,
+                const int32_t* plan, void* workspace, int64_t workspace_bytes, const void* q,
+                int64_t q_token_stride, const void* key_cache, const void* value_cache,
+                int64_t cache_block_stride, int64_t cache_token_stride, int64_t num_blocks,
+                const int32_t* indices, int64_t num_indices, float sm_scale, void* out,
+                int64_t out_token_stride, float* lse, void* stream) {
   KVC_REQUIRE(sched, KVC_ERR_INVALID_ARG, "null schedule");
+  const bool cut = split && split->num_parts > 0;
+  const bool parts = cut && workspace && workspace_bytes >= split->workspace_bytes;
   const int Hq = sched->num_qo_heads, Hkv = sched->num_kv_heads;
   KVC_REQUIRE(Hkv > 0 && Hq % Hkv == 0 && sched->head_dim == kD && sched->page_size == kPage &&
                   sched->tile_tokens == kTileRows / (Hq / Hkv) && sched->num_items >= 0 &&
-                  sched->plan_ints == plan_ints_for(sched->num_items, Hkv),
+                  (!cut || (split->num_units > 0 && split->num_merges > 0 &&
+                            split->base_offset == split_plan_ints(split->num_units,
+                                                                  split->num_merges) &&
+                            split->workspace_bytes ==
+                                int64_t(split->num_parts) * kTileRows * (kD + 1) * 4)) &&
+                  sched->plan_ints == (cut ? split->base_offset : 0) +
+                                          plan_ints_for(sched->num_items, Hkv),
               KVC_ERR_INVALID_ARG, "schedule not produced by kvc_prefill_plan");
+  KVC_REQUIRE(!parts || aligned(workspace, 16), KVC_ERR_ALIGNMENT,
+              "prefill workspace must be 16-byte aligned");
   if (sched->num_items == 0) return ok();
   KVC_REQUIRE(plan && q && key_cache && value_cache && out && indices, KVC_ERR_INVALID_ARG,
               "null pointer");
@@ -867,6 +1185,7 @@ extern "C" int kvc_batch_prefill_run(const kvc_prefill_schedule* sched, const in
                   cache_token_stride % 8 == 0,
               KVC_ERR_ALIGNMENT, "q/out/cache/plan must be 16-byte aligned with matching "
                                  "strides");
+  if (cut && !parts) plan += split->base_offset;
   PrefillArgs a;
   a.q = static_cast<const uint16_t*>(q);
   a.q_stride = q_token_stride;
@@ -877,7 +1196,8 @@ extern "C" int kvc_batch_prefill_run(const kvc_prefill_schedule* sched, const in
   a.num_blocks = num_blocks;
   a.indices = indices;
   a.num_indices = num_indices;
-  const int64_t workgroups = plan_workgroups(sched->num_items, Hkv);
+  const int64_t workgroups = parts ? std::min<int64_t>(kMaxWorkgroups, split->num_units)
+                                   : plan_workgroups(sched->num_items, Hkv);
   a.wg_units = reinterpret_cast<const int2*>(plan);
   a.units = reinterpret_cast<const int4*>(plan + plan_table_ints(workgroups));
   a.num_kv_heads = Hkv;
@@ -886,14 +1206,45 @@ extern "C" int kvc_batch_prefill_run(const kvc_prefill_schedule* sched, const in
   a.out = static_cast<uint16_t*>(out);
   a.out_stride = out_token_stride;
   a.lse = lse;
+  a.unit_part = parts ? plan + split->parts_offset : nullptr;
+  a.part_o = parts ? static_cast<float*>(workspace) : nullptr;
+  a.part_lse = parts ? a.part_o + int64_t(split->num_parts) * kTileRows * kD : nullptr;
+  const int4* merges = parts ? reinterpret_cast<const int4*>(plan + split->merges_offset) : nullptr;
+  const int num_merges = parts ? split->num_merges : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (Hq / Hkv) {
-    case 1: launch<1>(a, int(workgroups), s); break;
-    case 2: launch<2>(a, int(workgroups), s); break;
-    case 4: launch<4>(a, int(workgroups), s); break;
-    case 8: launch<8>(a, int(workgroups), s); break;
+    case 1: launch<1>(a, int(workgroups), merges, num_merges, s); break;
+    case 2: launch<2>(a, int(workgroups), merges, num_merges, s); break;
+    case 4: launch<4>(a, int(workgroups), merges, num_merges, s); break;
+    case 8: launch<8>(a, int(workgroups), merges, num_merges, s); break;
     default: KVC_REQUIRE(false, KVC_ERR_UNSUPPORTED, "group must be 1, 2, 4 or 8");
   }
   KVC_LAUNCH_CHECK();
   return ok();
+}
+
+}  // namespace
+
+extern "C" int kvc_batch_prefill_run(const kvc_prefill_schedule* sched, const int32_t* plan,
+                                     const void* q, int64_t q_token_stride,
+                                     const void* key_cache, const void* value_cache,
+                                     int64_t cache_block_stride, int64_t cache_token_stride,
+                                     int64_t num_blocks, const int32_t* indices,
+                                     int64_t num_indices, float sm_scale, void* out,
+                                     int64_t out_token_stride, float* lse, void* stream) {
+  return prefill_run(sched, nullptr, plan, nullptr, 0, q, q_token_stride, key_cache, value_cache,
+                     cache_block_stride, cache_token_stride, num_blocks, indices, num_indices,
+                     sm_scale, out, out_token_stride, lse, stream);
+}
+
+extern "C" int kvc_batch_prefill_split_run(
+    const kvc_prefill_schedule* sched, const kvc_prefill_split* split, const int32_t* plan,
+    void* workspace, int64_t workspace_bytes, const void* q, int64_t q_token_stride,
+    const void* key_cache, const void* value_cache, int64_t cache_block_stride,
+    int64_t cache_token_stride, int64_t num_blocks, const int32_t* indices, int64_t num_indices,
+    float sm_scale, void* out, int64_t out_token_stride, float* lse, void* stream) {
+  KVC_REQUIRE(split, KVC_ERR_INVALID_ARG, "null split");
+  return prefill_run(sched, split, plan, workspace, workspace_bytes, q, q_token_stride, key_cache,
+                     value_cache, cache_block_stride, cache_token_stride, num_blocks, indices,
+                     num_indices, sm_scale, out, out_token_stride, lse, stream);
 }

@@ -31,6 +31,10 @@ __all__ = ["BatchPrefillWithPagedKVCacheWrapper"]
 # and its most workgroups (one per CU; each runs a list of work items).
 _TILE_ROWS = 256
 _MAX_WORKGROUPS = 256
+# Batches of at most so many units may be cut along their keys, into at most so
+# many pieces (csrc/prefill.hip).
+_SPLIT_MAX_UNITS = 512
+_MAX_PIECES = 768
 
 
 def _fail(msg: str) -> None:
@@ -48,8 +52,10 @@ def _host_int32(t: torch.Tensor, n: int, name: str) -> np.ndarray:
 class BatchPrefillWithPagedKVCacheWrapper:
     """Prefill attention of multi-token queries over a paged KV cache ("NHD").
 
-    ``float_workspace_buffer`` only fixes the device (the kernel keeps no
-    split-K partials); it is accepted for interface parity.
+    ``float_workspace_buffer`` only fixes the device; it is accepted for
+    interface parity.  The partials of a batch whose long units are cut along
+    their keys live in a tensor of the call (a decode wrapper may share the
+    buffer on another stream).
     """
 
     def __init__(self, float_workspace_buffer: torch.Tensor, kv_layout: str = "NHD",
@@ -111,11 +117,9 @@ class BatchPrefillWithPagedKVCacheWrapper:
         q_lens = np.diff(qo.astype(np.int64)) if batch > 0 else np.zeros(0, np.int64)
         cap = self._plan_capacity(q_lens, group, num_kv_heads)
 
-        sched = _lib.KvcPrefillSchedule()
         hs = torch.empty(cap, dtype=torch.int32, pin_memory=True)
-        _lib.call("kvc_prefill_plan", qo.ctypes.data, kv.ctypes.data, lpl.ctypes.data, batch,
-                  num_qo_heads, num_kv_heads, head_dim_qk, page_size, 1 if causal else 0,
-                  sched, hs.data_ptr(), cap)
+        sched = self._schedule_into(qo, kv, lpl, batch, num_qo_heads, num_kv_heads, head_dim_qk,
+                                    page_size, causal, hs)
         self._plan_dev = hs[: max(sched.plan_ints, 8)].to(self._device, non_blocking=True)
         idx = paged_kv_indices[:total_pages]
         if idx.is_cuda:
@@ -137,22 +141,28 @@ class BatchPrefillWithPagedKVCacheWrapper:
     def _plan_capacity(q_lens: np.ndarray, group: int, num_kv_heads: int) -> int:
         """int32 entries to reserve for the plan image (16-byte multiple): the
         workgroups' (first unit, units) table, padded to 4 entries, and one
-        8-entry record per (query tile, KV head)."""
+        8-entry record per (query tile, KV head); for batches of few units
+        also what cutting them along their keys adds."""
         tile = _TILE_ROWS // group if group in (1, 2, 4, 8) else 1
         ql = np.maximum(np.asarray(q_lens, np.int64), 0)
         units = int(np.sum((ql + tile - 1) // tile)) * max(int(num_kv_heads), 1)
         table = (2 * min(_MAX_WORKGROUPS, units) + 3) // 4 * 4
+        if units <= _SPLIT_MAX_UNITS:
+            # a table, the pieces' records and partial indices, the tiles' merge
+            # records, and the plan of whole units after them
+            return 2 * _MAX_WORKGROUPS + 9 * _MAX_PIECES + 8 * units + table + 8 * units + 8
         return table + 8 * units + 8
 
     def _schedule_into(self, qo: np.ndarray, kv: np.ndarray, lpl: np.ndarray, batch: int,
                        num_qo_heads: int, num_kv_heads: int, head_dim: int, page_size: int,
                        causal: bool, image: torch.Tensor) -> _lib.KvcPrefillSchedule:
-        """kvc_prefill_plan into the pinned int32 ``image`` (sized by
-        ``_plan_capacity``)."""
+        """kvc_prefill_plan_split into the pinned int32 ``image`` (sized by
+        ``_plan_capacity``); the schedule carries its ``split``."""
         sched = _lib.KvcPrefillSchedule()
-        _lib.call("kvc_prefill_plan", qo.ctypes.data, kv.ctypes.data, lpl.ctypes.data, batch,
-                  num_qo_heads, num_kv_heads, head_dim, page_size, 1 if causal else 0,
-                  sched, image.data_ptr(), image.numel())
+        sched.split = _lib.KvcPrefillSplit()
+        _lib.call("kvc_prefill_plan_split", qo.ctypes.data, kv.ctypes.data, lpl.ctypes.data,
+                  batch, num_qo_heads, num_kv_heads, head_dim, page_size, 1 if causal else 0,
+                  sched, sched.split, image.data_ptr(), image.numel())
         return sched
 
     def _install(self, sched: _lib.KvcPrefillSchedule, plan_dev: torch.Tensor,
@@ -219,7 +229,17 @@ class BatchPrefillWithPagedKVCacheWrapper:
             _fail("lse must be contiguous float32 [total_q, num_qo_heads]")
         sh = (stream.cuda_stream if stream is not None
               else _lib.current_stream_handle(self._device))
-        _lib.call("kvc_batch_prefill_run", self._sched, self._plan_dev.data_ptr(),
+        ws, nbytes = None, int(self._sched.split.workspace_bytes)
+        if nbytes:
+            # from the pool of the stream that uses it, so that its memory is
+            # free there, and goes back there; a full card runs whole units
+            try:
+                with torch.cuda.stream(stream):
+                    ws = torch.empty(nbytes, dtype=torch.uint8, device=self._device)
+            except torch.cuda.OutOfMemoryError:
+                nbytes = 0
+        _lib.call("kvc_batch_prefill_split_run", self._sched, self._sched.split,
+                  self._plan_dev.data_ptr(), ws.data_ptr() if ws is not None else None, nbytes,
                   q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
                   k_cache.stride(0), k_cache.stride(1), k_cache.shape[0],
                   self._indices.data_ptr(), self._indices.numel(), self._sm_scale,

@@ -298,6 +298,37 @@ int kvc_prefill_plan(const int32_t* qo_indptr_host, const int32_t* kv_indptr_hos
                      kvc_prefill_schedule* schedule, int32_t* plan_host,
                      int64_t plan_capacity);
 
+/* The same plan with long units cut along their keys.  Where the batch's units
+ * leave CUs idle (few query tiles over long histories), units of more than 16
+ * key tiles are cut into pieces; the pieces of a (query tile, KV head) leave
+ * fp32 partials in a workspace and a second kernel merges them with the
+ * log-sum-exp rule.  num_parts 0: nothing was cut, the image and the results
+ * are kvc_prefill_plan's.  Otherwise schedule->plan_ints covers
+ *   the workgroups' table | num_units unit records | [parts_offset] num_units
+ *   partial indices (-1: writes the output) | [merges_offset] num_merges
+ *   records of 8 int32 (KV head, first output row, rows, first partial,
+ *   partials, 0, 0, 0) | [base_offset] kvc_prefill_plan's image
+ * and a cut unit's record counts kv_len and pages from its first key.
+ * kvc_batch_prefill_split_run takes workspace_bytes of device memory (16-byte
+ * aligned; its contents are not kept between calls); with none, or with less,
+ * it runs the whole units of base_offset. */
+typedef struct kvc_prefill_split {
+  int32_t num_units;
+  int32_t num_parts;
+  int32_t num_merges;
+  int32_t parts_offset;
+  int32_t merges_offset;
+  int32_t base_offset;
+  int64_t workspace_bytes;
+} kvc_prefill_split;
+
+int kvc_prefill_plan_split(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host,
+                           const int32_t* last_page_len_host, int32_t batch,
+                           int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim,
+                           int32_t page_size, int32_t causal,
+                           kvc_prefill_schedule* schedule, kvc_prefill_split* split,
+                           int32_t* plan_host, int64_t plan_capacity);
+
 /* q/out: [total_q][num_qo_heads][head_dim] with a token stride (elements).
  * q, out, the caches and the plan 16-byte aligned, every stride a multiple
  * of 8 elements (KVC_ERR_ALIGNMENT otherwise).  The cache's block stride
@@ -305,6 +336,15 @@ int kvc_prefill_plan(const int32_t* qo_indptr_host, const int32_t* kv_indptr_hos
  * 2 GiB: KVC_ERR_INVALID_ARG otherwise. */
 int kvc_batch_prefill_run(
     const kvc_prefill_schedule* schedule, const int32_t* plan,
+    const void* q, int64_t q_token_stride,
+    const void* key_cache, const void* value_cache,
+    int64_t cache_block_stride, int64_t cache_token_stride,
+    int64_t num_blocks, const int32_t* indices, int64_t num_indices,
+    float sm_scale, void* out, int64_t out_token_stride, float* lse, void* stream);
+
+int kvc_batch_prefill_split_run(
+    const kvc_prefill_schedule* schedule, const kvc_prefill_split* split,
+    const int32_t* plan, void* workspace, int64_t workspace_bytes,
     const void* q, int64_t q_token_stride,
     const void* key_cache, const void* value_cache,
     int64_t cache_block_stride, int64_t cache_token_stride,
