@@ -78,12 +78,14 @@ class KvcPrefillSplit(ctypes.Structure):
     """Mirror of ``kvc_prefill_split`` (include/kvc.h)."""
 
     _fields_ = [
+        ("num_workgroups", c_int32),
         ("num_units", c_int32),
         ("num_parts", c_int32),
         ("num_merges", c_int32),
         ("parts_offset", c_int32),
         ("merges_offset", c_int32),
         ("base_offset", c_int32),
+        ("reserved", c_int32),
         ("workspace_bytes", c_int64),
     ]
 

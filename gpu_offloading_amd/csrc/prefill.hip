@@ -733,30 +733,39 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_mfma_kernel(PrefillArgs a
   else run(std::integral_constant<int, 1>{});
 }
 
-// Merge of the split tiles: workgroup (tile x KV head, 16 of its 256 rows); 16
-// threads per row fold its partials, eight dims each, with the log-sum-exp rule.
-// Bound by latency: a few partials per row, read four at a time, all from L2 or
-// MALL where the pieces just left them.
+// Merge of the split tiles with the log-sum-exp rule: workgroup (tile x KV head,
+// 4 of its 256 rows), a wave per row; each quarter of the wave folds every fourth
+// partial, eight dims a lane, and two shuffles add the quarters.  Bound by
+// latency: a few partials per row, left in L2 or MALL just before, so a row has
+// up to 8 of them in flight.  3 tiles of one head with 80 partials per row: 39 us
+// with the pieces' kernel, 58 with 16 threads a row; 80 tiles with 3-5: 9-12 us
+// either way (40 MB of partials).
 // Record: (KV head, first output token, rows, first partial, partials, 0, 0, 0).
+constexpr int kMergeRows = 4;
 template <int G>
-__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, const int4* merges) {
+__global__ __launch_bounds__(64 * kMergeRows) void prefill_merge_kernel(PrefillArgs a,
+                                                                        const int4* merges) {
   const int4 rec = merges[2 * blockIdx.x];
   const int nparts = merges[2 * blockIdx.x + 1].x;
-  const int row = blockIdx.y * 16 + (threadIdx.x >> 4);
-  const int c = threadIdx.x & 15;
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.y * kMergeRows + (threadIdx.x >> 6);
+  const int c = lane & 15;
   if (row >= rec.z) return;
   const int64_t p0 = int64_t(rec.w) * kTileRows + row;
   float mx = -INFINITY;
-  for (int p = 0; p < nparts; ++p) mx = fmaxf(mx, a.part_lse[p0 + int64_t(p) * kTileRows]);
+  for (int p = lane; p < nparts; p += 64)
+    mx = fmaxf(mx, a.part_lse[p0 + int64_t(p) * kTileRows]);
+#pragma unroll
+  for (int x = 32; x; x >>= 1) mx = fmaxf(mx, __shfl_xor(mx, x));
   if (mx == -INFINITY) mx = 0.f;  // no key in any: weights 0 (and NaN where a partial is NaN)
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, S = 0.f;
-  constexpr int kAhead = 4;  // partials in flight per thread
-  for (int q0 = 0; q0 < nparts; q0 += kAhead) {
+  constexpr int kAhead = 2;  // partials in flight per quarter
+  for (int q0 = lane >> 4; q0 < nparts; q0 += 4 * kAhead) {
     float4 x[kAhead][2];
     float w[kAhead];
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
-      const int64_t pr = p0 + int64_t(min(q0 + i, nparts - 1)) * kTileRows;
+      const int64_t pr = p0 + int64_t(min(q0 + 4 * i, nparts - 1)) * kTileRows;
       const float4* src = reinterpret_cast<const float4*>(a.part_o + pr * kD + 8 * c);
       x[i][0] = src[0];
       x[i][1] = src[1];
@@ -764,7 +773,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, const
     }
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
-      if (q0 + i < nparts) {
+      if (q0 + 4 * i < nparts) {
         S += w[i];
         const float v[8] = {x[i][0].x, x[i][0].y, x[i][0].z, x[i][0].w,
                             x[i][1].x, x[i][1].y, x[i][1].z, x[i][1].w};
@@ -773,6 +782,13 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, const
       }
     }
   }
+#pragma unroll
+  for (int x = 16; x <= 32; x <<= 1) {
+    S += __shfl_xor(S, x);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] += __shfl_xor(acc[e], x);
+  }
+  if (lane >= 16) return;
   const float inv = S > 0.f ? 1.f / S : 0.f;
   const int64_t tok = rec.y + row / G;
   const int hq = rec.x * G + row % G;
@@ -794,7 +810,8 @@ void launch(const PrefillArgs& a, int workgroups, const int4* merges, int num_me
     return;
   }
   prefill_mfma_kernel<G, true><<<dim3(unsigned(workgroups)), kThreads, 0, s>>>(a);
-  prefill_merge_kernel<G><<<dim3(unsigned(num_merges), kTileRows / 16), 256, 0, s>>>(a, merges);
+  prefill_merge_kernel<G><<<dim3(unsigned(num_merges), kTileRows / kMergeRows), 64 * kMergeRows, 0,
+                                s>>>(a, merges);
 }
 
 // Persistent workgroups: at most one per CU of an MI355X (256), each running
@@ -810,20 +827,24 @@ int64_t plan_ints_for(int64_t items, int hkv) {
 // Split plans.  A batch of few query tiles over long histories has fewer units
 // than the chip has CUs, or a few long ones: 3 chunks of 60-400 tokens over
 // 3000-8000 tokens (8 KV heads, group 4) are 80 units of about 100 key tiles,
-// 157 us with 176 CUs idle.  Units are then cut into pieces of about `piece`
-// key tiles, which leave fp32 partials that a second kernel merges: 90 us; 3
-// chunks of 40 tokens over 25000-29000 tokens of one head 546 -> 54 us.  A unit
-// costs its key tiles + kUnitCost (its start and end, 4.6-6.4 us against 1.6 us
-// per tile) and the second launch kMergeCost; the plan takes the pieces that
-// end soonest by that, and whole units if none is a tenth sooner.  Units of up
-// to kSplitTiles tiles stay whole (the merge costs what cutting them gives), and
-// so do batches of more than kSplitMaxUnits units, which fill the chip.
+// 157 us with 176 CUs idle.  The units' key tiles are then dealt out in one
+// sequence, an equal share to each workgroup, cutting units at the shares' ends;
+// the pieces of a cut unit leave fp32 partials that a second kernel merges:
+// 77 us; 3 chunks of 40 tokens over 25000-29000 tokens of one head 546 -> 39 us.
+// (Equal pieces of each unit, longest first to the least loaded workgroup,
+// took 90 us: up to a piece's length is lost at the end, and 400 partials of
+// 131 KB are written and read where this leaves 300.)
+// A unit or piece costs its key tiles + kUnitCost (its start and end, 4.6-6.4 us
+// against 1.6 us per tile) and the second launch kMergeCost; units stay whole
+// unless cutting them is a tenth sooner by that.  Units of up to kSplitTiles
+// tiles are never cut (with units of 11 on cut, a prefill of 1100 tokens took
+// 37.8 us against 33.7), and batches of more than kSplitMaxUnits units fill the
+// chip as they are.
 constexpr int kSplitTiles = 16;
 constexpr int kMinPiece = 4;       // tiles; shorter ones are mostly start and end
 constexpr int kUnitCost = 4;
 constexpr int kMergeCost = 5;       // the merge launch, in tiles
 constexpr int64_t kSplitMaxUnits = 512;
-constexpr int64_t kMaxPieces = 768;  // units of a split plan: at most 101 MB of partials
 
 // End of the longest workgroup when units of these costs are dealt longest
 // first to the least loaded of W workgroups.
@@ -841,60 +862,79 @@ int64_t makespan(std::vector<int>& costs, int64_t W) {
   return end;
 }
 
-int pieces_of(int tiles, int piece) {
-  return tiles > kSplitTiles ? (tiles + piece - 1) / piece : 1;
+// A piece of unit (item, KV head): `tiles` key tiles from `first` on, the unit's
+// index-th.
+struct Piece {
+  int64_t item;
+  int head, first, tiles, index;
+};
+
+// Deals the units' key tiles out in order, up to `share` cost per workgroup (a
+// little more where the rest of a unit would be shorter than kMinPiece).
+// Consecutive workgroups get consecutive tiles, head by head: the query tiles of
+// one request and head are near each other.  Returns the largest cost, or -1 if
+// kMaxWorkgroups are too few.
+int64_t deal(const std::vector<int32_t>& rec, int64_t n, int hkv, int64_t share,
+             std::vector<std::vector<Piece>>* lists) {
+  int64_t w = 0, load = 0, most = 0;
+  if (lists) lists->assign(1, {});
+  auto next = [&]() {
+    ++w;
+    load = 0;
+    if (lists) lists->emplace_back();
+  };
+  for (int h = 0; h < hkv; ++h)
+    for (int64_t i = 0; i < n; ++i) {
+      int left = rec[i * kItemInts + 6], first = 0, index = 0;
+      const bool whole = left <= kSplitTiles;
+      do {  // a unit without keys is dealt, too
+        if (load > 0 && share - load - kUnitCost < (whole ? left : kMinPiece)) next();
+        const int64_t room = share - load - kUnitCost;
+        int take = whole ? left : int(std::min<int64_t>(left, std::max<int64_t>(room, kMinPiece)));
+        if (left - take < kMinPiece) take = left;
+        if (lists) lists->back().push_back(Piece{i, h, first, take, index});
+        load += take + kUnitCost;
+        most = std::max(most, load);
+        if (w >= kMaxWorkgroups) return -1;
+        left -= take;
+        first += take;
+        ++index;
+      } while (left > 0);
+    }
+  return most;
 }
 
-// Key tiles per piece that end a batch of these units soonest, or 0 to leave
+// The workgroups' share that ends a batch of these units soonest, or 0 to leave
 // them whole (unless splitting saves a tenth).
-int split_piece(const std::vector<int32_t>& rec, int64_t n, int hkv) {
+int64_t split_share(const std::vector<int32_t>& rec, int64_t n, int hkv) {
   if (n * hkv > kSplitMaxUnits) return 0;
   int64_t total = 0;
   int longest = 0;
   std::vector<int> costs;
   for (int64_t i = 0; i < n; ++i) {
     const int t = rec[i * kItemInts + 6];
-    total += int64_t(t) * hkv;
+    total += int64_t(t + kUnitCost) * hkv;
     longest = std::max(longest, t);
     costs.insert(costs.end(), size_t(hkv), t + kUnitCost);
   }
   if (longest <= kSplitTiles) return 0;
-  const int64_t share = (total + n * hkv * kUnitCost) / kMaxWorkgroups;
   const int64_t whole = makespan(costs, kMaxWorkgroups);
-  if (whole <= share + share / 8) return 0;
-  int best = 0;
-  int64_t best_end = whole - whole / 10;
-  int last = 0;
-  // Pieces of two workgroups' shares of all tiles, of one, of two thirds of one
-  // and of half of one.
-  for (int k = 1; k <= 4; ++k) {
-    const int piece = int(std::max<int64_t>(kMinPiece, (2 * total + k * kMaxWorkgroups - 1) /
-                                                           (k * kMaxWorkgroups)));
-    if (piece == last || piece >= longest) continue;
-    last = piece;
-    costs.clear();
-    for (int64_t i = 0; i < n; ++i) {
-      const int t = rec[i * kItemInts + 6];
-      const int np = pieces_of(t, piece);
-      for (int x = 0; x < np; ++x)
-        costs.insert(costs.end(), size_t(hkv),
-                     int(int64_t(t) * (x + 1) / np - int64_t(t) * x / np) + kUnitCost);
-    }
-    if (int64_t(costs.size()) > kMaxPieces) continue;
-    const int64_t end = makespan(costs, kMaxWorkgroups) + kMergeCost;
-    if (end < best_end) {
-      best_end = end;
-      best = piece;
-    }
+  int64_t lo = std::max<int64_t>(total / kMaxWorkgroups, kMinPiece + kUnitCost), hi = whole;
+  if (lo + kMergeCost >= whole - whole / 10) return 0;
+  while (lo < hi) {  // the least share that kMaxWorkgroups can hold
+    const int64_t mid = lo + (hi - lo) / 2;
+    if (deal(rec, n, hkv, mid, nullptr) >= 0) hi = mid;
+    else lo = mid + 1;
   }
-  return best;
+  const int64_t most = deal(rec, n, hkv, lo, nullptr);
+  return most >= 0 && most + kMergeCost < whole - whole / 10 ? lo : 0;
 }
 
 // int32 entries of a split plan's image: the workgroups' table, the unit
 // records, each unit's partial (padded to 4) and the merge records.
-int64_t split_plan_ints(int64_t units, int64_t merges) {
-  return plan_table_ints(std::min(kMaxWorkgroups, units)) + units * kItemInts +
-         (units + 3) / 4 * 4 + merges * kItemInts;
+int64_t split_plan_ints(int64_t workgroups, int64_t units, int64_t merges) {
+  return plan_table_ints(workgroups) + units * kItemInts + (units + 3) / 4 * 4 +
+         merges * kItemInts;
 }
 
 // The plan of whole units: plan_ints_for(n, hkv) entries.
@@ -944,40 +984,28 @@ void write_plan(const std::vector<int32_t>& rec, int64_t n, int hkv, int32_t* pl
   }
 }
 
-int split_plan(const std::vector<int32_t>& rec, int64_t n, int hkv, int piece, int tile_tokens,
-               int group, kvc_prefill_schedule* sched, kvc_prefill_split* split,
-               int32_t* plan_host, int64_t plan_capacity) {
-  struct Piece {
-    int64_t item;
-    int first, tiles, index;   // key tiles; index within its tile's pieces
-  };
-  std::vector<Piece> pieces;   // of one KV head
-  std::vector<int> count(static_cast<size_t>(n));
-  int64_t split_items = 0;
-  for (int64_t i = 0; i < n; ++i) {
-    const int t = rec[i * kItemInts + 6];
-    const int np = pieces_of(t, piece);
-    count[size_t(i)] = np;
-    split_items += np > 1;
-    for (int x = 0; x < np; ++x) {
-      const int t0 = int(int64_t(t) * x / np), t1 = int(int64_t(t) * (x + 1) / np);
-      pieces.push_back(Piece{i, t0, t1 - t0, x});
-    }
+int split_plan(const std::vector<int32_t>& rec, int64_t n, int hkv, int64_t share,
+               int tile_tokens, int group, kvc_prefill_schedule* sched,
+               kvc_prefill_split* split, int32_t* plan_host, int64_t plan_capacity) {
+  std::vector<std::vector<Piece>> lists;
+  deal(rec, n, hkv, share, &lists);
+  const int64_t W = int64_t(lists.size());
+  std::vector<int> count(size_t(n * hkv)), first_part(size_t(n * hkv));
+  int64_t units = 0, parts = 0, merges = 0;
+  for (const auto& l : lists) {
+    units += int64_t(l.size());
+    for (const Piece& p : l) ++count[size_t(p.head * n + p.item)];
   }
-  const int64_t per_head = int64_t(pieces.size()), units = per_head * hkv;
-  const int64_t merges = split_items * hkv, W = std::min(kMaxWorkgroups, units);
-  std::vector<int64_t> first(static_cast<size_t>(n), -1);  // partial of piece 0, per head 0
-  int64_t parts = 0;
-  for (int64_t i = 0; i < n; ++i)
-    if (count[size_t(i)] > 1) {
-      first[size_t(i)] = parts;
-      parts += count[size_t(i)];
+  for (size_t u = 0; u < count.size(); ++u)
+    if (count[u] > 1) {
+      first_part[u] = int(parts);
+      parts += count[u];
+      ++merges;
     }
-  const int64_t parts_per_head = parts;
-  parts *= hkv;
   const int64_t table = plan_table_ints(W);
-  const int64_t base = split_plan_ints(units, merges);
+  const int64_t base = split_plan_ints(W, units, merges);
   sched->plan_ints = base + plan_ints_for(n, hkv);
+  split->num_workgroups = int32_t(W);
   split->num_units = int32_t(units);
   split->num_parts = int32_t(parts);
   split->num_merges = int32_t(merges);
@@ -987,54 +1015,39 @@ int split_plan(const std::vector<int32_t>& rec, int64_t n, int hkv, int piece, i
   split->workspace_bytes = parts * kTileRows * (kD + 1) * 4;
   KVC_REQUIRE(plan_host && plan_capacity >= sched->plan_ints, KVC_ERR_WORKSPACE,
               "plan buffer too small: need " + std::to_string(sched->plan_ints) + " int32");
-  // Longest first, to the least loaded workgroup.
-  std::vector<int64_t> order(static_cast<size_t>(units));
-  for (int64_t u = 0; u < units; ++u) order[size_t(u)] = u;
-  auto key = [&](int64_t u) { return pieces[size_t(u % per_head)]; };
-  std::stable_sort(order.begin(), order.end(),
-                   [&](int64_t x, int64_t y) { return key(x).tiles > key(y).tiles; });
-  std::vector<std::vector<int64_t>> lists(static_cast<size_t>(W));
-  typedef std::pair<int64_t, int64_t> Slot;  // (load, workgroup)
-  std::priority_queue<Slot, std::vector<Slot>, std::greater<Slot>> free_at;
-  for (int64_t b = 0; b < W; ++b) free_at.push(Slot(0, b));
-  for (const int64_t u : order) {
-    const Slot sl = free_at.top();
-    free_at.pop();
-    lists[size_t(sl.second)].push_back(u);
-    free_at.push(Slot(sl.first + key(u).tiles + kUnitCost, sl.second));
-  }
   std::fill_n(plan_host, table, 0);
   int32_t* unit_part = plan_host + split->parts_offset;
   std::fill(unit_part, plan_host + split->merges_offset, -1);
   int64_t next = 0;
   for (int64_t b = 0; b < W; ++b) {
+    // Workgroup b runs on XCD b % 8: its workgroups take neighbouring lists,
+    // which read the same requests' K and V through one L2.
+    const int64_t x = b % 8, per = W / 8, more = W % 8;
+    const auto& list = lists[size_t(x * per + std::min(x, more) + b / 8)];
     plan_host[2 * b] = int32_t(next);
-    plan_host[2 * b + 1] = int32_t(lists[size_t(b)].size());
-    for (const int64_t u : lists[size_t(b)]) {
-      const Piece p = key(u);
-      const int64_t head = u / per_head;
+    plan_host[2 * b + 1] = int32_t(list.size());
+    for (const Piece& p : list) {
+      const size_t u = size_t(p.head * n + p.item);
       int32_t* dst = plan_host + table + next * kItemInts;
       std::copy_n(rec.data() + p.item * kItemInts, kItemInts, dst);
       const int pages = std::min<int>(dst[7], p.first * (kKeys / kPage));
-      dst[0] = int32_t(head);
+      dst[0] = p.head;
       dst[3] -= p.first * kKeys;   // keys from the piece's first on
       dst[5] += pages;
       dst[6] = p.tiles;
       dst[7] -= pages;
-      if (count[size_t(p.item)] > 1)
-        unit_part[next] = int32_t(head * parts_per_head + first[size_t(p.item)] + p.index);
+      if (count[u] > 1) unit_part[next] = first_part[u] + p.index;
       ++next;
     }
   }
   int32_t* m = plan_host + split->merges_offset;
-  for (int64_t head = 0; head < hkv; ++head)
+  for (int h = 0; h < hkv; ++h)
     for (int64_t i = 0; i < n; ++i) {
-      if (count[size_t(i)] <= 1) continue;
+      const size_t u = size_t(h * n + i);
+      if (count[u] <= 1) continue;
       const int32_t* r = rec.data() + i * kItemInts;
-      const int32_t out[kItemInts] = {int32_t(head), r[4] + r[1],
-                                      std::min(tile_tokens, r[2] - r[1]) * group,
-                                      int32_t(head * parts_per_head + first[size_t(i)]),
-                                      count[size_t(i)], 0, 0, 0};
+      const int32_t out[kItemInts] = {h, r[4] + r[1], std::min(tile_tokens, r[2] - r[1]) * group,
+                                      first_part[u], count[u], 0, 0, 0};
       m = std::copy_n(out, kItemInts, m);
     }
   write_plan(rec, n, hkv, plan_host + base);
@@ -1100,10 +1113,11 @@ int prefill_plan(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host,
   sched->plan_ints = plan_ints_for(n, num_kv_heads);
   if (split) {
     *split = kvc_prefill_split{};
+    split->num_workgroups = int32_t(plan_workgroups(n, num_kv_heads));
     split->num_units = int32_t(n * num_kv_heads);
-    const int piece = split_piece(rec, n, num_kv_heads);
-    if (piece > 0)
-      return split_plan(rec, n, num_kv_heads, piece, tile_tokens, group, sched, split, plan_host,
+    const int64_t share = split_share(rec, n, num_kv_heads);
+    if (share > 0)
+      return split_plan(rec, n, num_kv_heads, share, tile_tokens, group, sched, split, plan_host,
                         plan_capacity);
   }
   KVC_REQUIRE(plan_host && plan_capacity >= sched->plan_ints, KVC_ERR_WORKSPACE,
@@ -1155,7 +1169,10 @@ int prefill_run(const kvc_prefill_schedule* sched, const kvc_prefill_split* spli
   KVC_REQUIRE(Hkv > 0 && Hq % Hkv == 0 && sched->head_dim == kD && sched->page_size == kPage &&
                   sched->tile_tokens == kTileRows / (Hq / Hkv) && sched->num_items >= 0 &&
                   (!cut || (split->num_units > 0 && split->num_merges > 0 &&
-                            split->base_offset == split_plan_ints(split->num_units,
+                            split->num_workgroups > 0 &&
+                            split->num_workgroups <= kMaxWorkgroups &&
+                            split->base_offset == split_plan_ints(split->num_workgroups,
+                                                                  split->num_units,
                                                                   split->num_merges) &&
                             split->workspace_bytes ==
                                 int64_t(split->num_parts) * kTileRows * (kD + 1) * 4)) &&
@@ -1196,7 +1213,7 @@ int prefill_run(const kvc_prefill_schedule* sched, const kvc_prefill_split* spli
   a.num_blocks = num_blocks;
   a.indices = indices;
   a.num_indices = num_indices;
-  const int64_t workgroups = parts ? std::min<int64_t>(kMaxWorkgroups, split->num_units)
+  const int64_t workgroups = parts ? split->num_workgroups
                                    : plan_workgroups(sched->num_items, Hkv);
   a.wg_units = reinterpret_cast<const int2*>(plan);
   a.units = reinterpret_cast<const int4*>(plan + plan_table_ints(workgroups));

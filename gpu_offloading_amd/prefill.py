@@ -31,10 +31,10 @@ __all__ = ["BatchPrefillWithPagedKVCacheWrapper"]
 # and its most workgroups (one per CU; each runs a list of work items).
 _TILE_ROWS = 256
 _MAX_WORKGROUPS = 256
-# Batches of at most so many units may be cut along their keys, into at most so
-# many pieces (csrc/prefill.hip).
+# Batches of at most so many units may be cut along their keys, once at each
+# workgroup's end at most (csrc/prefill.hip).
 _SPLIT_MAX_UNITS = 512
-_MAX_PIECES = 768
+_MAX_PIECES = _SPLIT_MAX_UNITS + _MAX_WORKGROUPS
 
 
 def _fail(msg: str) -> None:

@@ -304,7 +304,7 @@ int kvc_prefill_plan(const int32_t* qo_indptr_host, const int32_t* kv_indptr_hos
  * fp32 partials in a workspace and a second kernel merges them with the
  * log-sum-exp rule.  num_parts 0: nothing was cut, the image and the results
  * are kvc_prefill_plan's.  Otherwise schedule->plan_ints covers
- *   the workgroups' table | num_units unit records | [parts_offset] num_units
+ *   num_workgroups' table | num_units unit records | [parts_offset] num_units
  *   partial indices (-1: writes the output) | [merges_offset] num_merges
  *   records of 8 int32 (KV head, first output row, rows, first partial,
  *   partials, 0, 0, 0) | [base_offset] kvc_prefill_plan's image
@@ -313,12 +313,14 @@ int kvc_prefill_plan(const int32_t* qo_indptr_host, const int32_t* kv_indptr_hos
  * aligned; its contents are not kept between calls); with none, or with less,
  * it runs the whole units of base_offset. */
 typedef struct kvc_prefill_split {
+  int32_t num_workgroups;
   int32_t num_units;
   int32_t num_parts;
   int32_t num_merges;
   int32_t parts_offset;
   int32_t merges_offset;
   int32_t base_offset;
+  int32_t reserved;
   int64_t workspace_bytes;
 } kvc_prefill_split;
 

@@ -36,9 +36,10 @@ def _plan(q_lens, kv_lens, group, hkv, causal):
     return image(None), image(split), split
 
 
-def _units(sched, img, num_units):
-    table = (2 * min(256, num_units) + 3) // 4 * 4
-    return img[table:table + 8 * num_units].reshape(-1, 8), img[:2 * min(256, num_units)]
+def _units(img, num_units, workgroups):
+    table = (2 * workgroups + 3) // 4 * 4
+    return (img[table:table + 8 * num_units].reshape(-1, 8),
+            img[:2 * workgroups].reshape(-1, 2))
 
 
 @pytest.mark.parametrize("q_lens,kv_lens,group,hkv,causal,cut", [
@@ -47,6 +48,7 @@ def _units(sched, img, num_units):
     ([700], [1400], 4, 8, 0, True),
     ([40] * 9, [3000 + 77 * i for i in range(9)], 1, 4, 1, True),
     ([256 * 16], [256 * 16], 1, 32, 1, False),      # 512 units, balanced as they are
+    ([40] + [64] * 20, [9000] + [0] * 20, 4, 8, 1, True),   # units without keys
     ([257 * 2], [30000], 1, 32, 1, True),
     ([300], [30000], 1, 32, 1, True),
     ([1024], [1024], 4, 8, 1, False),               # 16 key tiles: never cut
@@ -64,9 +66,9 @@ def test_split_plan_covers_every_key_once(q_lens, kv_lens, group, hkv, causal, c
         assert not cut
         return
     assert cut
-    whole, _ = _units(base, base_img, n)
-    rec, wg = _units(sched, img, split.num_units)
-    wg = wg.reshape(-1, 2)
+    whole, _ = _units(base_img, n, min(256, n))
+    assert split.num_workgroups <= 256
+    rec, wg = _units(img, split.num_units, split.num_workgroups)
     assert np.array_equal(wg[:, 0], np.concatenate([[0], np.cumsum(wg[:-1, 1])]))
     assert wg[:, 1].min() >= 1 and wg[:, 1].sum() == split.num_units
     part = img[split.parts_offset:split.parts_offset + split.num_units]
