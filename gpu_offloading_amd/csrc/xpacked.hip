@@ -8,18 +8,25 @@
 // head_size 128, block_size 16.
 //
 // In this layout one (block, head) is a contiguous 4 KB of K and 4 KB of V,
-// so decode streams straight into registers, no LDS staging:
-//   q.k : lane (token t = l%16, chunk group cg = l/16) loads the 16-byte
-//         chunks 4cg..4cg+3 of token t (dims 32cg..32cg+31), 16 dot2 per query
-//         head, then two xor-shuffles sum the 4 chunk groups;
-//   p.v : lane l loads 16 B at 16l + 1024j (dim l/2 + 32j, tokens 8(l%2) ..
-//         +7; every load one contiguous KB); p is rounded to the cache dtype
-//         in (t, t+1) pairs -- as vLLM's kernel does before its value dot --
-//         broadcast with v_readlane and folded with 4 dot2 per dim; lanes l
-//         and l^1 add their token halves at the end.
+// so decode streams straight into the operand registers of
+// v_mfma_f32_16x16x32 (lane l = row or column l%16, k = 8(l/16) .. +7), two
+// pages at a time, no LDS staging:
+//   q.k : A = K, rows = the 16 tokens of a page; lane l's 16-byte chunk
+//         4i + l/16 of token l%16, i < 4, is one contiguous KB per load.  B = Q,
+//         columns = the query heads of the KV head, zero beyond the group.  A
+//         lane gets head l%16's scores of tokens 4(l/16) .. +3 of each page.
+//   p.v : A = V, rows = 16 head dims, k = page l/32's tokens 8(l/16%2) .. +7:
+//         16 bytes per lane, two 512-byte runs per load.  B = p, rounded to the
+//         cache dtype -- as vLLM's kernel does before its value dot; two lane
+//         swaps turn the score layout into it.  A lane gets head l%16's
+//         dims 16j + 4(l/16) .. +3.
+// With one query head per KV head 15 of 16 columns are idle, and the matrix
+// cores still have time to spare: 16 MFMAs per 16 KB of K and V.  (With dot2 on
+// the vector units the group's heads were work of their own: 6 sequences of
+// 16400-19000, 4 KV heads, group 8, 111 us; now 48, at 4.7 TB/s.)
 // Block ids are loaded 64 pages at a time, one per lane, and broadcast.
-// A workgroup (4 waves) owns one KV head x one 512-token partition (v2) or the
-// whole sequence (v1); wave w takes pages w, w+4, ...; the waves' softmax
+// A workgroup owns one KV head x one 512-token partition (v2) or the whole
+// sequence (v1); wave w of W takes page pairs w, w+W, ...; the waves' softmax
 // states are merged through LDS.  v2 leaves vLLM's per-partition max logit,
 // exp-sum and normalised partial output, and a reduce kernel combines them.
 #include "kvc_common.h"
@@ -30,10 +37,14 @@
 namespace kvc {
 namespace {
 
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-
 constexpr int kThreads = 256;
-constexpr int kV2Waves = 4;  // waves per v2 workgroup (1, 2 and 4 measured alike)
+// Waves per v2 workgroup.  164 registers let a CU hold three 4-wave workgroups or
+// one of 8 waves.  A grid of many rounds per CU reads faster through the latter
+// (64 sequences of 512-4096, 32 heads, 16384 workgroups: 355 us against 367),
+// fewer reads in flight each of neighbouring pages; a few rounds want the
+// overlap of several workgroups (6 of 16400-19000, 4 KV heads, 912: 48 against 53).
+constexpr int kV2Waves = 4, kV2WavesMany = 8;
+constexpr int64_t kManyWorkgroups = 4096;
 constexpr int kBlock = 16;    // tokens per block
 constexpr int kD = 128;       // head size
 constexpr int kX = 8;         // elements per 16-byte chunk
@@ -41,13 +52,18 @@ constexpr int kPart = 512;    // tokens per v2 partition (vLLM's)
 constexpr float kLn2 = 0.69314718055994530942f;
 constexpr float kLog2e = 1.44269504088896340736f;
 
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
 template <bool kBf16>
-__device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
+__device__ __forceinline__ f32x4_t mfma(uint4 a, uint4 b, f32x4_t c) {
   if constexpr (kBf16)
-    return dot2_bf16(a, b, c);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
   else
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, a),
-                                  __builtin_bit_cast(half2_t, b), c, false);
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a),
+                                                  __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
 }
 
 // float -> element bits, round to nearest even.
@@ -178,135 +194,143 @@ __global__ __launch_bounds__(64 * kW) void xpacked_decode_kernel(XDecodeArgs a) 
   const int t_end = kV1 ? seq_len : min(seq_len, t_begin + kPart);
   if (!kV1 && t_begin >= seq_len) return;  // the reduce never reads it
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int t = lane & 15, cg = lane >> 4;
+  const int r16 = lane & 15, grp = lane >> 4;
   const int Hq = a.num_kv_heads * G;
 
-  uint32_t qw[G][16];  // dims 32cg .. 32cg+31 of each query head, as pairs
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const uint16_t* qp = a.q + int64_t(b) * a.q_stride + int64_t(h * G + g) * kD + 32 * cg;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint4 v = reinterpret_cast<const uint4*>(qp)[i];
-      qw[g][4 * i] = v.x; qw[g][4 * i + 1] = v.y; qw[g][4 * i + 2] = v.z; qw[g][4 * i + 3] = v.w;
-    }
-  }
-  float m[G], l[G], acc[G][4];  // acc[g][j]: dim lane/2 + 32j, half of the tokens
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    m[g] = kNegBig;
-    l[g] = 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[g][j] = 0.f;
-  }
-
+  // This wave's page pairs: wave + kW*j, j < n_pairs.  Their block ids are
+  // loaded 64 at a time, one per lane, and broadcast with v_readlane.
   const int p_begin = t_begin / kBlock, p_end = (t_end + kBlock - 1) / kBlock;
   const int32_t* bt = a.block_tables + int64_t(b) * a.bt_stride;
-  // This wave's pages: p_begin + wave + 4j, j < n_pages.  Their block ids
-  // are loaded 64 at a time, one per lane, and broadcast with v_readlane.
-  const int first = p_begin + wave;
-  const int n_pages = p_end > first ? (p_end - first + kW - 1) / kW : 0;
+  const int pairs = (p_end - p_begin + 1) / 2;
+  const int n_pairs = pairs > wave ? (pairs - wave + kW - 1) / kW : 0;
+  auto page_of = [&](int j) { return p_begin + 2 * (wave + kW * j); };
   int32_t id_reg = -1;
-  auto id_at = [&](int jj) __attribute__((always_inline)) {
-    if ((jj & 63) == 0) {
-      const int p = first + kW * (jj + lane);
-      const int32_t id = (jj + lane < n_pages && p < a.bt_cols) ? bt[p] : -1;
-      id_reg = (id >= 0 && id < a.num_blocks) ? id : -1;
-    }
-    return __builtin_amdgcn_readlane(id_reg, jj & 63);
+  auto load_ids = [&](int j) __attribute__((always_inline)) {  // pairs j .. j+31
+    const int p = page_of(j + (lane >> 1)) + (lane & 1);
+    const int32_t id = p < min(p_end, a.bt_cols) ? bt[p] : -1;
+    id_reg = (id >= 0 && id < a.num_blocks) ? id : -1;
   };
-  // V of a (block, head) is [D][16 tokens]; lane l loads bytes 16l + 1024j,
-  // i.e. dim l/2 + 32j, tokens 8(l%2) .. +7 -- one contiguous KB per load.
-  struct Regs { uint4 k[4], v[4]; };
-  const int vt0 = 8 * (lane & 1);
-  auto load = [&](Regs& r, int32_t id) __attribute__((always_inline)) {
-    const int64_t base = int64_t(id < 0 ? 0 : id) * a.block_stride + int64_t(h) * a.head_stride;
-    const uint16_t* kb = a.k_cache + base + (int64_t(4 * cg) * kBlock + t) * kX;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r.k[i] = load_stream(kb + i * kBlock * kX);
-    const uint16_t* vb = a.v_cache + base + lane * kX;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) r.v[j] = load_stream(vb + j * 64 * kX);
-  };
-  auto consume = [&](Regs& r, int p, int32_t id) __attribute__((always_inline)) {
-    const int valid = id < 0 ? 0 : min(kBlock, t_end - p * kBlock);
-    uint32_t* vw = reinterpret_cast<uint32_t*>(r.v);  // [dim j][token pair k]
-    if (valid < kBlock) {
-      // tokens past the end: zero their V halves (they may hold NaN bits)
-#pragma unroll
-      for (int w = 0; w < 16; ++w) {
-        const int tok = vt0 + 2 * (w & 3);
-        vw[w] &= (tok < valid ? 0xffffu : 0u) | (tok + 1 < valid ? 0xffff0000u : 0u);
-      }
-    }
-    const bool live = t < valid;
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      float d = 0.f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        d = dot2<kBf16>(qw[g][4 * i + 0], r.k[i].x, d);
-        d = dot2<kBf16>(qw[g][4 * i + 1], r.k[i].y, d);
-        d = dot2<kBf16>(qw[g][4 * i + 2], r.k[i].z, d);
-        d = dot2<kBf16>(qw[g][4 * i + 3], r.k[i].w, d);
-      }
-      d += __shfl_xor(d, 16);
-      d += __shfl_xor(d, 32);
-      const float s = live ? d * a.scale_log2 : kNegBig;
-      const float m_new = fmaxf(m[g], row16_max(s));
-      const float pr = live ? fast_exp2(s - m_new) : 0.f;
-      const float alpha = fast_exp2(m[g] - m_new);
-      l[g] = fmaf(l[g], alpha, row16_sum(pr));
-      m[g] = m_new;
-      // (p[t], p[t+1]) as one element pair in even lanes, broadcast; this
-      // lane needs the pairs of tokens vt0 .. vt0+7.
-      const float nxt = __shfl_down(pr, 1, 16);
-      const uint32_t pair = to_elem<kBf16>(pr) | (to_elem<kBf16>(nxt) << 16);
-      uint32_t pw[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t lo = __builtin_amdgcn_readlane(pair, 2 * k);
-        const uint32_t hi = __builtin_amdgcn_readlane(pair, 8 + 2 * k);
-        pw[k] = vt0 ? hi : lo;
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float o = acc[g][j] * alpha;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) o = dot2<kBf16>(pw[k], vw[4 * j + k], o);
-        acc[g][j] = o;
-      }
-    }
-  };
+  if (n_pairs > 0) load_ids(0);
 
-  // Two register stages: the wave's next page is in flight while one is consumed.
-  Regs ra, rb;
-  int32_t ida = -1, idb = -1;
-  if (n_pages > 0) { ida = id_at(0); load(ra, ida); }
-  for (int j = 0; j < n_pages; j += 2) {
-    if (j + 1 < n_pages) { idb = id_at(j + 1); load(rb, idb); }
-    consume(ra, first + kW * j, ida);
-    if (j + 1 >= n_pages) break;
-    if (j + 2 < n_pages) { ida = id_at(j + 2); load(ra, ida); }
-    consume(rb, first + kW * (j + 1), idb);
+  uint4 qw[4];  // head r16's dims 32i + 8grp .. +7
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    qw[i] = r16 < G ? *reinterpret_cast<const uint4*>(a.q + int64_t(b) * a.q_stride +
+                                                      int64_t(h * G + r16) * kD + 32 * i + 8 * grp)
+                    : make_uint4(0, 0, 0, 0);
+
+  float m = kNegBig, l = 0.f;  // of head r16; l of this lane's tokens only
+  f32x4_t acc[8];              // dims 16j + 4grp .. +3 of head r16
+#pragma unroll
+  for (int j = 0; j < 8; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  const uint16_t* kh = a.k_cache + int64_t(h) * a.head_stride + lane * kX;
+  const uint16_t* vh =
+      a.v_cache + int64_t(h) * a.head_stride + r16 * kBlock + 8 * (grp & 1);
+  for (int j = 0; j < n_pairs; ++j) {
+    if (j > 0 && (j & 31) == 0) load_ids(j);
+    const int32_t id0 = __builtin_amdgcn_readlane(id_reg, 2 * (j & 31));
+    const int32_t id1 = __builtin_amdgcn_readlane(id_reg, 2 * (j & 31) + 1);
+    uint4 k[2][4], v[8];
+    const uint16_t* k0 = kh + int64_t(max(id0, 0)) * a.block_stride;
+    const uint16_t* k1 = kh + int64_t(max(id1, 0)) * a.block_stride;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      k[0][i] = load_stream(k0 + i * 64 * kX);
+      k[1][i] = load_stream(k1 + i * 64 * kX);
+    }
+    const int32_t idv = lane < 32 ? id0 : id1;
+    const uint16_t* vb = vh + int64_t(max(idv, 0)) * a.block_stride;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = load_stream(vb + i * 16 * kBlock);
+
+    const int left = t_end - page_of(j) * kBlock;  // tokens from the pair's first on
+    const int valid0 = id0 < 0 ? 0 : left, valid1 = id1 < 0 ? 0 : left - kBlock;
+    f32x4_t s[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      s[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[x] = mfma<kBf16>(k[x][i], qw[i], s[x]);
+    }
+    float mx = m;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const bool live = 4 * grp + r < (x ? valid1 : valid0);
+        s[x][r] = live ? s[x][r] * a.scale_log2 : kNegBig;
+        mx = fmaxf(mx, s[x][r]);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float alpha = fast_exp2(m - mx);
+    m = mx;
+    float sum = 0.f;
+    uint32_t pw[2][2];  // [page][token pair]
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      float p[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const bool live = 4 * grp + r < (x ? valid1 : valid0);
+        p[r] = live ? fast_exp2(s[x][r] - mx) : 0.f;
+        sum += p[r];
+      }
+#pragma unroll
+      for (int w = 0; w < 2; ++w)
+        pw[x][w] = to_elem<kBf16>(p[2 * w]) | (to_elem<kBf16>(p[2 * w + 1]) << 16);
+    }
+    l = fmaf(l, alpha, sum);
+    // Lane group g holds tokens 4g .. +3 of both pages and needs tokens 8(g%2)
+    // .. +7 of page g/2: swap the upper half of page 0 with the lower of page
+    // 1, then the odd groups of the one with the even ones of the other.
+    uint32_t po[4];
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      const auto x = __builtin_amdgcn_permlane32_swap(pw[0][w], pw[1][w], false, false);
+      const auto y = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
+      po[w] = y[0];
+      po[2 + w] = y[1];
+    }
+    const uint4 pb = make_uint4(po[0], po[1], po[2], po[3]);
+    if (min(valid0, valid1) < kBlock) {
+      // tokens past the end or of a missing page: zero V (it may hold NaN bits)
+      const int valid = (lane < 32 ? valid0 : valid1) - 8 * (grp & 1);
+      uint32_t mask[4];
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+        mask[w] = (2 * w < valid ? 0xffffu : 0u) | (2 * w + 1 < valid ? 0xffff0000u : 0u);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        v[i].x &= mask[0];
+        v[i].y &= mask[1];
+        v[i].z &= mask[2];
+        v[i].w &= mask[3];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i][e] *= alpha;
+      acc[i] = mfma<kBf16>(v[i], pb, acc[i]);
+    }
   }
-  // the two token halves of each dim live in lanes l and l^1
-#pragma unroll
-  for (int g = 0; g < G; ++g)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[g][j] += __shfl_xor(acc[g][j], 1);
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
 
-  // Merge the 4 waves' states.
+  // Merge the waves' states.
   __shared__ float s_m[kW][G], s_l[kW][G];
-  __shared__ float s_acc[kW][G][kD];
-  if (lane == 0)
+  __shared__ __align__(16) float s_acc[kW][G][kD];
+  if (r16 < G) {
+    if (grp == 0) {
+      s_m[wave][r16] = m;
+      s_l[wave][r16] = l;
+    }
 #pragma unroll
-    for (int g = 0; g < G; ++g) { s_m[wave][g] = m[g]; s_l[wave][g] = l[g]; }
-  if ((lane & 1) == 0)
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) s_acc[wave][g][(lane >> 1) + 32 * j] = acc[g][j];
+    for (int i = 0; i < 8; ++i)
+      *reinterpret_cast<f32x4_t*>(&s_acc[wave][r16][16 * i + 4 * grp]) = acc[i];
+  }
   __syncthreads();
   // Thread j < G*D: head g = j / D, dim d = j % D.
   for (int j = threadIdx.x; j < G * kD; j += 64 * kW) {
@@ -411,10 +435,15 @@ __global__ __launch_bounds__(kRedThreads) void xpacked_reduce_kernel(XDecodeArgs
 template <int G, bool kBf16>
 void launch_decode(const XDecodeArgs& a, bool v1, int parts, int hkv, int seqs, hipStream_t s) {
   if (v1) {
-    xpacked_decode_kernel<G, kBf16, true, 4><<<dim3(hkv, seqs, 1), 256, 0, s>>>(a);
+    // 8 waves: a workgroup has the whole sequence (4 sequences of 300-2000, 8 KV
+    // heads, group 4: 20 us, with 4 waves 23; 32 of 300-900, 32 heads: 59 and 64).
+    xpacked_decode_kernel<G, kBf16, true, 8><<<dim3(hkv, seqs, 1), 64 * 8, 0, s>>>(a);
   } else {
-    xpacked_decode_kernel<G, kBf16, false, kV2Waves>
-        <<<dim3(hkv, seqs, parts), 64 * kV2Waves, 0, s>>>(a);
+    const dim3 grid(hkv, seqs, parts);
+    if (int64_t(hkv) * seqs * parts >= kManyWorkgroups)
+      xpacked_decode_kernel<G, kBf16, false, kV2WavesMany><<<grid, 64 * kV2WavesMany, 0, s>>>(a);
+    else
+      xpacked_decode_kernel<G, kBf16, false, kV2Waves><<<grid, 64 * kV2Waves, 0, s>>>(a);
     xpacked_reduce_kernel<kBf16><<<dim3(hkv * G, seqs), kRedThreads, 0, s>>>(a);
   }
 }
