@@ -54,24 +54,28 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _check_cuda(*ts: torch.Tensor) -> torch.device:
-    dev = None
+    # By device index: comparing torch.device objects costs three times that.
+    first, index = None, -1
     for t in ts:
         if t is None:
             continue
         if not t.is_cuda:
             _fail(f"expected a GPU tensor, got one on {t.device}")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            _fail(f"tensors on different devices: {dev} vs {t.device}")
-    return dev
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
+            _fail(f"tensors on different devices: {first.device} vs {t.device}")
+    return None if first is None else first.device
 
 
-def _check_cache(cache: torch.Tensor, name: str) -> None:
-    if cache.dim() != 4:
-        _fail(f"{name} must be [num_blocks, block_size, num_kv_heads, head_dim], got {tuple(cache.shape)}")
-    if cache.stride(3) != 1 or cache.stride(2) != cache.shape[3]:
-        _fail(f"{name}: the heads of a token must be contiguous (strides {cache.stride()})")
+def _check_cache(cache: torch.Tensor, name: str):
+    """[nb, bs, H, D] with packed heads; returns its shape and strides."""
+    shape, st = cache.shape, cache.stride()
+    if len(shape) != 4:
+        _fail(f"{name} must be [num_blocks, block_size, num_kv_heads, head_dim], got {tuple(shape)}")
+    if st[3] != 1 or st[2] != shape[3]:
+        _fail(f"{name}: the heads of a token must be contiguous (strides {st})")
+    return shape, st
 
 
 def _oob_ptr(oob_count: Optional[torch.Tensor]) -> Optional[int]:
@@ -104,30 +108,30 @@ def reshape_and_cache_flash(key: torch.Tensor, value: torch.Tensor,
     if kv_cache_dtype != "auto":
         _fail(f"kv_cache_dtype={kv_cache_dtype!r} is not supported (only 'auto')")
     dev = _check_cuda(key, value, key_cache, value_cache, slot_mapping)
-    _check_cache(key_cache, "key_cache")
-    _check_cache(value_cache, "value_cache")
-    if key_cache.shape != value_cache.shape or key_cache.stride() != value_cache.stride():
+    shape, cs = _check_cache(key_cache, "key_cache")
+    if (shape, cs) != _check_cache(value_cache, "value_cache"):
         _fail("key_cache and value_cache must have the same shape and strides")
-    if key.dtype != key_cache.dtype or value.dtype != value_cache.dtype:
+    if key.dtype is not key_cache.dtype or value.dtype is not value_cache.dtype:
         _fail(f"dtype mismatch: key {key.dtype} vs cache {key_cache.dtype}")
-    if slot_mapping.dtype != torch.int64 or slot_mapping.dim() != 1:
+    if slot_mapping.dtype is not torch.int64 or slot_mapping.dim() != 1:
         _fail("slot_mapping must be a 1-D int64 tensor")
     if not slot_mapping.is_contiguous():
         _fail("slot_mapping must be contiguous")
-    nb, bs, h, d = key_cache.shape
+    nb, bs, h, d = shape
     n = slot_mapping.numel()
-    for name, t in (("key", key), ("value", value)):
-        if t.dim() != 3 or t.shape[1] != h or t.shape[2] != d:
-            _fail(f"{name} must be [num_tokens, {h}, {d}], got {tuple(t.shape)}")
-        if t.shape[0] < n:
-            _fail(f"{name} has {t.shape[0]} rows but slot_mapping has {n}")
-        if t.stride(2) != 1 or t.stride(1) != d:
-            _fail(f"{name}: heads of a token must be contiguous (strides {t.stride()})")
+    ks, vs = key.stride(), value.stride()
+    for name, t, st in (("key", key, ks), ("value", value, vs)):
+        ts = t.shape
+        if len(ts) != 3 or ts[1] != h or ts[2] != d:
+            _fail(f"{name} must be [num_tokens, {h}, {d}], got {tuple(ts)}")
+        if ts[0] < n:
+            _fail(f"{name} has {ts[0]} rows but slot_mapping has {n}")
+        if st[2] != 1 or st[1] != d:
+            _fail(f"{name}: heads of a token must be contiguous (strides {st})")
     _lib.call("kvc_reshape_and_cache_flash",
               key.data_ptr(), value.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(),
               slot_mapping.data_ptr(), n, h, d, bs, nb, key_cache.element_size(),
-              key.stride(0), value.stride(0), key_cache.stride(0), key_cache.stride(1),
-              _oob_ptr(oob_count), _stream_handle(dev, stream))
+              ks[0], vs[0], cs[0], cs[1], _oob_ptr(oob_count), _stream_handle(dev, stream))
 
 
 # --------------------------------------------------------------------------
@@ -474,21 +478,24 @@ _XDTYPES = {torch.float16: 0, torch.bfloat16: 1}
 
 def _check_xpacked(key_cache: torch.Tensor, value_cache: torch.Tensor):
     """[nb, H, D/x, bs, x] and [nb, H, D, bs] with packed inner dimensions
-    and equal block / head strides; returns (nb, H, D, bs, x)."""
-    if key_cache.dim() != 5 or value_cache.dim() != 4:
+    and equal block / head strides; returns (nb, H, D, bs, x), the block and
+    head strides and the dtype."""
+    kshape, vshape = key_cache.shape, value_cache.shape
+    if len(kshape) != 5 or len(vshape) != 4:
         _fail("x-packed caches must be key [nb, H, D/x, bs, x] and value [nb, H, D, bs]")
-    nb, h, dx, bs, x = key_cache.shape
+    nb, h, dx, bs, x = kshape
     d = dx * x
-    if tuple(value_cache.shape) != (nb, h, d, bs):
-        _fail(f"value_cache must be [{nb}, {h}, {d}, {bs}], got {tuple(value_cache.shape)}")
-    if key_cache.dtype not in _XDTYPES or value_cache.dtype != key_cache.dtype:
+    if vshape != (nb, h, d, bs):
+        _fail(f"value_cache must be [{nb}, {h}, {d}, {bs}], got {tuple(vshape)}")
+    dt = key_cache.dtype
+    if dt not in _XDTYPES or value_cache.dtype is not dt:
         _fail("x-packed caches must be float16 or bfloat16, both the same")
-    if x != 16 // key_cache.element_size():
-        _fail(f"x must be 16 bytes / element = {16 // key_cache.element_size()}, got {x}")
-    if (key_cache.stride()[2:] != (bs * x, x, 1) or value_cache.stride()[2:] != (bs, 1)
-            or key_cache.stride()[:2] != value_cache.stride()[:2]):
+    if x != 8:  # both types have 2 bytes
+        _fail(f"x must be 16 bytes / element = 8, got {x}")
+    bst, hst, s2, s3, s4 = key_cache.stride()
+    if (s2, s3, s4) != (bs * x, x, 1) or value_cache.stride() != (bst, hst, bs, 1):
         _fail("x-packed caches: inner dimensions packed, block/head strides equal for K and V")
-    return nb, h, d, bs, x
+    return nb, h, d, bs, x, bst, hst, dt
 
 
 def reshape_and_cache(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor,
@@ -505,19 +512,21 @@ def reshape_and_cache(key: torch.Tensor, value: torch.Tensor, key_cache: torch.T
     if kv_cache_dtype != "auto":
         _fail(f"kv_cache_dtype={kv_cache_dtype!r} is not supported (only 'auto')")
     dev = _check_cuda(key, value, key_cache, value_cache, slot_mapping)
-    nb, h, d, bs, x = _check_xpacked(key_cache, value_cache)
-    if slot_mapping.dtype != torch.int64 or slot_mapping.dim() != 1 or not slot_mapping.is_contiguous():
+    nb, h, d, bs, x, bst, hst, dt = _check_xpacked(key_cache, value_cache)
+    if slot_mapping.dtype is not torch.int64 or slot_mapping.dim() != 1 or not slot_mapping.is_contiguous():
         _fail("slot_mapping must be a contiguous 1-D int64 tensor")
     n = slot_mapping.numel()
-    for name, t in (("key", key), ("value", value)):
-        if t.dim() != 3 or tuple(t.shape[1:]) != (h, d) or t.shape[0] < n:
-            _fail(f"{name} must be [>= {n}, {h}, {d}], got {tuple(t.shape)}")
-        if t.stride(2) != 1 or t.stride(1) != d or t.dtype != key_cache.dtype:
+    ks, vs = key.stride(), value.stride()
+    for name, t, st in (("key", key, ks), ("value", value, vs)):
+        ts = t.shape
+        if len(ts) != 3 or ts[1] != h or ts[2] != d or ts[0] < n:
+            _fail(f"{name} must be [>= {n}, {h}, {d}], got {tuple(ts)}")
+        if st[2] != 1 or st[1] != d or t.dtype is not dt:
             _fail(f"{name}: heads must be packed and the dtype must match the cache")
     _lib.call("kvc_reshape_and_cache_xpacked", key.data_ptr(), value.data_ptr(),
               key_cache.data_ptr(), value_cache.data_ptr(), slot_mapping.data_ptr(), n, h, d,
-              bs, x, nb, key.stride(0), value.stride(0), key_cache.stride(0),
-              key_cache.stride(1), _oob_ptr(oob_count), _stream_handle(dev, stream))
+              bs, x, nb, ks[0], vs[0], bst, hst, _oob_ptr(oob_count),
+              _stream_handle(dev, stream))
 
 
 def _paged_attention(v2: bool, out, exp_sums, max_logits, tmp_out, query, key_cache,
@@ -534,41 +543,42 @@ def _paged_attention(v2: bool, out, exp_sums, max_logits, tmp_out, query, key_ca
             _fail("k/v scales other than 1.0 are not supported (no fp8 cache)")
     dev = _check_cuda(out, query, key_cache, value_cache, block_tables, seq_lens,
                       exp_sums, max_logits, tmp_out)
-    nb, hkv, d, bs, x = _check_xpacked(key_cache, value_cache)
+    nb, hkv, d, bs, _, bst, hst, dt = _check_xpacked(key_cache, value_cache)
     if hkv != num_kv_heads:
         _fail(f"num_kv_heads={num_kv_heads} but the cache holds {hkv} heads")
     if block_size != bs:
         _fail(f"block_size={block_size} but the cache blocks hold {bs} tokens")
-    if query.dim() != 3 or query.shape[2] != d or query.dtype != key_cache.dtype:
+    qs, qt = query.shape, query.stride()
+    if len(qs) != 3 or qs[2] != d or query.dtype is not dt:
         _fail(f"query must be [num_seqs, num_heads, {d}] of the cache dtype")
-    seqs, hq = query.shape[0], query.shape[1]
-    if query.stride(2) != 1 or query.stride(1) != d:
+    seqs, hq = qs[0], qs[1]
+    if qt[2] != 1 or qt[1] != d:
         _fail("query: heads must be packed")
-    if tuple(out.shape) != (seqs, hq, d) or not out.is_contiguous() or out.dtype != query.dtype:
+    if out.shape != qs or not out.is_contiguous() or out.dtype is not dt:
         _fail(f"out must be a contiguous [{seqs}, {hq}, {d}] tensor of the query dtype")
-    if block_tables.dtype != torch.int32 or block_tables.dim() != 2 or block_tables.stride(1) != 1:
+    ts, tt = block_tables.shape, block_tables.stride()
+    if block_tables.dtype is not torch.int32 or len(ts) != 2 or tt[1] != 1:
         _fail("block_tables must be int32 [num_seqs, max_blocks] with packed rows")
-    if block_tables.shape[0] < seqs or seq_lens.dtype != torch.int32 or seq_lens.numel() < seqs:
+    if ts[0] < seqs or seq_lens.dtype is not torch.int32 or seq_lens.numel() < seqs:
         _fail("block_tables / seq_lens need one row / entry per sequence")
     if not seq_lens.is_contiguous():
         _fail("seq_lens must be contiguous")
-    dt = _XDTYPES[key_cache.dtype]
-    common = (query.data_ptr(), query.stride(0), key_cache.data_ptr(), value_cache.data_ptr(),
+    common = (query.data_ptr(), qt[0], key_cache.data_ptr(), value_cache.data_ptr(),
               seqs, hq, num_kv_heads, d, float(scale), block_tables.data_ptr(),
-              block_tables.stride(0), block_tables.shape[1], seq_lens.data_ptr(), bs,
-              int(max_seq_len), nb, dt, key_cache.stride(0), key_cache.stride(1),
-              _stream_handle(dev, stream))
+              tt[0], ts[1], seq_lens.data_ptr(), bs, int(max_seq_len), nb, _XDTYPES[dt],
+              bst, hst, _stream_handle(dev, stream))
     if not v2:
         _lib.call("kvc_paged_attention_v1", out.data_ptr(), *common)
         return
-    parts = exp_sums.shape[-1] if exp_sums.dim() == 3 else 0
+    es = exp_sums.shape
+    parts = es[2] if len(es) == 3 else 0
     for name, t, shp in (("exp_sums", exp_sums, (seqs, hq, parts)),
                          ("max_logits", max_logits, (seqs, hq, parts)),
                          ("tmp_out", tmp_out, (seqs, hq, parts, d))):
-        if tuple(t.shape) != shp or not t.is_contiguous():
+        if t.shape != shp or not t.is_contiguous():
             _fail(f"{name} must be a contiguous {shp} tensor")
-    if exp_sums.dtype != torch.float32 or max_logits.dtype != torch.float32 \
-            or tmp_out.dtype != query.dtype:
+    if exp_sums.dtype is not torch.float32 or max_logits.dtype is not torch.float32 \
+            or tmp_out.dtype is not dt:
         _fail("exp_sums / max_logits are float32, tmp_out has the query dtype")
     _lib.call("kvc_paged_attention_v2", out.data_ptr(), exp_sums.data_ptr(),
               max_logits.data_ptr(), tmp_out.data_ptr(), parts, *common)
