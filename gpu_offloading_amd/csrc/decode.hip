@@ -790,7 +790,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void decode_small_kernel(DecodeAr
 // small: K and V go from memory into registers, nothing is staged in LDS, and
 // no barrier sits in the page loop.  A workgroup's waves are its KV heads times
 // TS page shares: wave (head, ts) streams units ts, ts + TS, ... of the
-// segment (a unit is one page, at head_dim 64 two).  One unit is in flight per
+// segment (a unit is one page, at head_dim 64 below group 8 two).  One unit is in flight per
 // wave while another is consumed -- K's registers are refilled as soon as q.k
 // has read them, V's after p.v -- and 8 to 16 waves per CU hide the latency.
 // Every K and V load of the wave reads whole token rows (four rows of 256 B at
@@ -815,7 +815,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void decode_small_kernel(DecodeAr
 // its time), us:
 //   32 requests of 500-3001 tokens, 8 KV heads, group 8, head_dim 64: 63.8 -> 32.5
 //   64 of 512-4096, group 8, head_dim 128: 133 -> 101 (5.6 TB/s)
-//   64 of 512-4096, one KV head, group 4, head_dim 128: 35.6 -> 21.0
+//   64 of 512-4096, one KV head, group 4, head_dim 128: 35.6 -> 20.1
 //   32 of 500-3000, 8 KV heads, head_dim 256, group 4: 93 -> 80 (5.7 TB/s)
 //   32 of 500-3000, 16 KV heads, head_dim 64, group 1: 47.9 -> 44.8
 // ---------------------------------------------------------------------------
@@ -838,9 +838,17 @@ constexpr int kNonTemporal = 2;
 template <int G, int D>
 struct WaveCfg {
   static_assert(G <= 4 || D < 256, "four query heads per wave at head_dim 256");
-  // Waves per workgroup: as many as a CU's registers hold.
+  // Waves per workgroup.  At head_dim 64 and 256 as many as registers allow
+  // without spills, at most 16 (12 for groups 2 and 4 at 64: 16 took 16.8 ->
+  // 19.0 us on 64 requests of one KV head, 8 took 17.2).  At head_dim 128 a
+  // page is 8 KB per wave, so eight waves have 64 KB in flight, enough for the
+  // CU's share of HBM; more only start later and meet in more states at a
+  // piece's end.  16 waves at group 1 or 12 else -> 8, one layer, us:
+  //   64 requests of 512-4096, one KV head: group 1 21.0 -> 18.7, 4 21.2 -> 20.4,
+  //   8 24.9 -> 24.1; 8 of 300-2000, 8 heads: group 4 16.0 -> 15.1, 8 22.2 -> 21.2;
+  //   one of 32000: 29.6 -> 28.8.  (16 at groups 2 and 4: 1 to 15% slower than 12.)
   static constexpr int kWaves =
-      G == 1 ? (D == 256 ? 12 : 16) : (D == 256 ? 8 : 12);
+      D == 256 ? (G == 1 ? 12 : 8) : D == 128 ? 8 : (G == 1 ? 16 : 12);
   static constexpr int kPages = D == 64 && G < 8 ? 2 : 1;  // pages a wave takes at a time
   static constexpr int kGroups = G == 8 ? 2 : 1;   // query heads in fours
   static constexpr int kGroupHeads = G < 4 ? G : 4;
@@ -1834,6 +1842,7 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
   //     8 x 68  18.3 -> 15.0 / 15.5 / 16.7     16 x 110  30.9 -> 30.3 / 28.9 / 28.3
   //     20 x 37 19.9 -> 19.2 / 18.6 / 18.6     60 x 27   28.8 -> 30.2 / 27.9 / 27.6
   //     12 x 14 12.5 -> 13.2 / 12.5 / 12.4     32 x 128  51.1 -> 55.0 / 51.7 / 50.7
+  //   (wave kernel with 12 waves; with the 8 it has now 8 x 68 takes 1 us less)
   //   groups 1, 2 (the LDS kernel's arithmetic is a quarter or half of that):
   //     2 x 138 18.3 -> 13.3 / 12.9 / 14.9     4 x 131   16.6 -> 16.4 / 15.5 / 16.0
   //     8 x 72  14.7 -> 16.2 / 15.4 / 14.8     20 x 37   16.6 -> 19.2 / 17.9 / 17.4
