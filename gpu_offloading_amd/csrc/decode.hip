@@ -1256,6 +1256,10 @@ __global__ __launch_bounds__((64 * WaveCfg<G, D>::kWaves), (WaveCfg<G, D>::kWave
           }
         }
         // Sum over the chunks of a row; lane row c keeps tokens t_row .. +3.
+        // The quads of a row must end up with the same bits, as they decide alone
+        // on the rescale and share the row's l: turned by two quads first, quads j
+        // and j + 2 hold the same sum, and turned by one then, every quad adds the
+        // same two.  (By one first, the quads' sums differ by fp32 rounding.)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           float x;
@@ -1263,8 +1267,8 @@ __global__ __launch_bounds__((64 * WaveCfg<G, D>::kWaves), (WaveCfg<G, D>::kWave
             x = swap16_add(d[0][r], d[1][r]);
           else
             x = swap16_add(swap32_add(d[0][r], d[2][r]), swap32_add(d[1][r], d[3][r]));
-          x += dpp<kDppRowRor4>(x);
           x += dpp<kDppRowRor8>(x);
+          x += dpp<kDppRowRor4>(x);
           p[g][y][r] = x;
         }
       }
