@@ -1743,6 +1743,12 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
   // kMaxSegPages pages each, at least one page each.  When the page cap
   // forces more segments than there are slots, the count is rounded
   // up to whole rounds of slots, so no round runs a few stragglers alone.
+  // A round of the wave kernel has no more workgroups than slots: one fills a CU
+  // (at head_dim 64 and 256 and for groups of 8), so of the 258 that 3, 6 or 12
+  // KV heads gave rounded up, two ran a second full length alone (32 requests of
+  // 500-3000 tokens, rounded up -> down, us: 6 heads, head_dim 64, group 4 31.9 ->
+  // 24.1; 6 at 256 103 -> 71; 6 at 128, group 8 66 -> 44; 3 at 64 26.4 -> 19.7).
+  // The LDS kernel's count stays rounded up (24 KV heads: 258).
   const int64_t slots = num_cus > 0 ? num_cus : 256;
   auto segment_count = [&](int heads) -> int64_t {
     if (total == 0) return 0;
@@ -1752,7 +1758,8 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
       n = std::max<int64_t>(num_segments_hint, at_least);
     } else {
       const int64_t groups = int64_t(num_kv_heads / heads) * q_splits;
-      const int64_t per_round = (slots + groups - 1) / groups;
+      const int64_t per_round = heads == kLdsHeads ? (slots + groups - 1) / groups
+                                                   : std::max<int64_t>(1, slots / groups);
       n = (std::max(per_round, at_least) + per_round - 1) / per_round * per_round;
     }
     return std::min<int64_t>(n, total);
