@@ -807,9 +807,10 @@ __global__ __launch_bounds__(64 * kSmallWaves) void decode_small_kernel(DecodeAr
 //   p.v : v_mfma_f32_4x4x1_16b_f32 with p in fp32 as it lies in the lanes and
 //         V widened to fp32 (exact): lane l holds eight dims of its row's token
 //         for the four heads.  A group of one multiplies on the VALU instead.
-// At a piece's end the rows' states are merged in the wave, then the TS waves'
-// through LDS with one barrier, and the piece is written.  Uniform plan records
-// come by scalar loads, which the loads in flight do not delay.
+// At a piece's end the rows' states are merged in the wave, then (a piece of more
+// than one unit) the TS waves' through LDS with one barrier, and the piece is
+// written.  Uniform plan records come by scalar loads, which the loads in flight
+// do not delay.
 //
 // One layer with its append (start: the kernel it replaces with the merge of
 // its time), us:
@@ -1073,9 +1074,16 @@ __global__ __launch_bounds__((64 * WaveCfg<G, D>::kWaves), (WaveCfg<G, D>::kWave
   };
 
   int parity = 0;
-  // Close piece k: the four rows' states of every wave are merged, then (TS > 1)
-  // those of the waves that shared the piece, and the piece is written.
+  bool holds = false;  // this wave has consumed pages of the piece (uniform)
+  // Close piece k: the four rows' states of every wave are merged, then those of
+  // the waves that shared the piece, and the piece is written.  A piece of one
+  // unit is written by the wave that holds it, and the others go on: no barrier.
+  // (Every wave closing every piece together cost about 2 us a piece: 40 requests
+  // of 3 tokens before 30 of 1590, 8 KV heads, group 4, head_dim 64 took 49.5 us,
+  // now 33.7; group 8 at 128 79 -> 51.)
   auto finish = [&]() __attribute__((always_inline)) {
+    const bool alone = (cp.y - g0) / PU == (cp.z - 1 - g0) / PU;  // the same in every wave
+    if (alone && !holds) return;
     const int fl = local_lane();
     const int c = fl >> 4, nn = fl & 15, v_chunk = D == 64 ? nn & 7 : nn;
 #pragma unroll
@@ -1104,7 +1112,7 @@ __global__ __launch_bounds__((64 * WaveCfg<G, D>::kWaves), (WaveCfg<G, D>::kWave
       }
       const float Lc = __shfl(L, c), Mc = __shfl(M, c);
       const int gl = 4 * g + c, gq = G * split + gl;  // query head of the workgroup, of the KV head
-      if (TS == 1) {
+      if (alone) {
         if (c < C::kGroupHeads) {
           const float inv = Lc > 0.f ? 1.f / Lc : 0.f;
 #pragma unroll
@@ -1131,9 +1139,9 @@ __global__ __launch_bounds__((64 * WaveCfg<G, D>::kWaves), (WaveCfg<G, D>::kWave
         }
       }
     }
-    if (TS > 1) {
+    if (!alone) {
       // One barrier per piece: the other parity's buffers are only written
-      // again after the next piece's barrier.
+      // again after the next such piece's barrier.
       lds_barrier();
       for (int i = 64 * wave + fl; i < hpw * G * (D / 2); i += 64 * W) {
         const int d = 2 * (i % (D / 2)), r = i / (D / 2);
@@ -1226,7 +1234,9 @@ __global__ __launch_bounds__((64 * WaveCfg<G, D>::kWaves), (WaveCfg<G, D>::kWave
         for (int x = 0; x < C::kQ; ++x) q[g][x] = qn[g][x];
       load_q(qn, scalar_int4(a.pieces, 2 * min(k + 1, k_end - 1)).x);
       reset();
+      holds = false;
     }
+    holds = true;
     // The tokens of each page that the piece holds: none of a missing page, or
     // of one that lies in another piece (a unit may cross into the next piece:
     // it is then consumed once for each, and refilled after the last).
