@@ -64,6 +64,8 @@ namespace {
 
 constexpr int kPage = 16;      // tokens per page (the engine's page_size)
 constexpr int kLdsHeads = 8;   // KV heads per workgroup of the LDS kernel
+constexpr int kMaxWaveHeads = 4;   // KV heads per workgroup of the wave kernel, at most
+constexpr int64_t kChipCus = 256;  // an MI355X's CUs
 constexpr int kIdRegs = 2;     // page-id registers per lane
 constexpr int kMaxSegPages = 64 * kIdRegs;
 constexpr int kReadGroup = 4;  // LDS reads scheduled together
@@ -833,6 +835,10 @@ typedef u32x4_t u32x4_a4_t __attribute__((aligned(4)));
 constexpr int kBufferRsrcWord3 = 0x00020000;
 constexpr int kNonTemporal = 2;
 
+constexpr int wave_kernel_waves(int group, int head_dim) {
+  return head_dim == 256 ? (group == 1 ? 12 : 8) : head_dim == 128 ? 8 : (group == 1 ? 16 : 12);
+}
+
 // G: query heads of a KV head that one workgroup serves.  At head_dim 256 a
 // group of 8 is served as two workgroups of four (q_splits 2): its accumulators
 // alone would fill a wave's registers.
@@ -848,8 +854,7 @@ struct WaveCfg {
   //   64 requests of 512-4096, one KV head: group 1 21.0 -> 18.7, 4 21.2 -> 20.4,
   //   8 24.9 -> 24.1; 8 of 300-2000, 8 heads: group 4 16.0 -> 15.1, 8 22.2 -> 21.2;
   //   one of 32000: 29.6 -> 28.8.  (16 at groups 2 and 4: 1 to 15% slower than 12.)
-  static constexpr int kWaves =
-      D == 256 ? (G == 1 ? 12 : 8) : D == 128 ? 8 : (G == 1 ? 16 : 12);
+  static constexpr int kWaves = wave_kernel_waves(G, D);
   static constexpr int kPages = D == 64 && G < 8 ? 2 : 1;  // pages a wave takes at a time
   static constexpr int kGroups = G == 8 ? 2 : 1;   // query heads in fours
   static constexpr int kGroupHeads = G < 4 ? G : 4;
@@ -936,8 +941,10 @@ __device__ __forceinline__ float quad_lane(float x) {
   return dpp<V * 0x55>(x);
 }
 
-template <int G, int D>
-__global__ __launch_bounds__((64 * WaveCfg<G, D>::kWaves), (WaveCfg<G, D>::kWaves / 4)) void decode_wave_kernel(DecodeArgs a) {
+// kNarrow: a workgroup is one wave per head, each streaming the whole segment.
+template <int G, int D, bool kNarrow>
+__global__ __launch_bounds__((64 * (kNarrow ? kMaxWaveHeads : WaveCfg<G, D>::kWaves)),
+                             (WaveCfg<G, D>::kWaves / 4)) void decode_wave_kernel(DecodeArgs a) {
   using C = WaveCfg<G, D>;
   constexpr int W = C::kWaves, NG = C::kGroups, NL = C::kLoads, NE = C::kDims, PU = C::kPages;
   __shared__ float s_o[2][W][G][D];
@@ -946,7 +953,8 @@ __global__ __launch_bounds__((64 * WaveCfg<G, D>::kWaves), (WaveCfg<G, D>::kWave
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int hpw = a.heads_per_group;
-  const int hw = wave % hpw, ts = wave / hpw, TS = W / hpw;
+  const int hw = kNarrow ? wave : wave % hpw, ts = kNarrow ? 0 : wave / hpw;
+  const int TS = kNarrow ? 1 : W / hpw;
   const int split = blockIdx.y % a.q_splits, h0 = blockIdx.y / a.q_splits * hpw;
   const int h = h0 + hw;
   const int group = G * a.q_splits;  // query heads of a KV head
@@ -1082,8 +1090,8 @@ __global__ __launch_bounds__((64 * WaveCfg<G, D>::kWaves), (WaveCfg<G, D>::kWave
   // of 3 tokens before 30 of 1590, 8 KV heads, group 4, head_dim 64 took 49.5 us,
   // now 33.7; group 8 at 128 79 -> 51.)
   auto finish = [&]() __attribute__((always_inline)) {
-    const bool alone = (cp.y - g0) / PU == (cp.z - 1 - g0) / PU;  // the same in every wave
-    if (alone && !holds) return;
+    const bool alone = kNarrow || (cp.y - g0) / PU == (cp.z - 1 - g0) / PU;  // the same in every wave
+    if (!kNarrow && alone && !holds) return;
     const int fl = local_lane();
     const int c = fl >> 4, nn = fl & 15, v_chunk = D == 64 ? nn & 7 : nn;
 #pragma unroll
@@ -1419,6 +1427,7 @@ __device__ __forceinline__ float wave_sum(float v) {
 // null): then no partial is read, and every request counts at most one
 // piece.
 constexpr int kSpecParts = 16;
+constexpr int64_t kNarrowPerCu = 8;  // narrow segments per CU, at most
 
 template <int D>
 __global__ __launch_bounds__(64) void decode_merge_kernel(MergeArgs a) {
@@ -1623,6 +1632,20 @@ std::vector<int64_t> cut_segments(const int32_t* indptr, int batch, int64_t tota
   return cut;
 }
 
+// The most segments that one request lies in.
+int32_t most_pieces(const int32_t* indptr, int batch, const std::vector<int64_t>& cut) {
+  int64_t most = 1;
+  size_t s = 1;
+  for (int b = 0; b < batch; ++b) {
+    while (s + 1 < cut.size() && cut[s] <= indptr[b]) ++s;  // the first cut past its start
+    size_t e = s;
+    while (e + 1 < cut.size() && cut[e] < indptr[b + 1]) ++e;
+    most = std::max<int64_t>(most, int64_t(e - s) + 1);
+    s = e;
+  }
+  return int32_t(most);
+}
+
 // Whether a head layout has the LDS kernel.
 bool lds_layout(int group, int head_dim, int num_kv_heads) {
   return head_dim == 128 && group <= 4 && num_kv_heads % kLdsHeads == 0;
@@ -1642,6 +1665,23 @@ bool valid_heads_per_group(int group, int head_dim, int num_kv_heads, int hpw) {
   return (hpw == 1 || hpw == 2 || hpw == 4) && num_kv_heads % hpw == 0;
 }
 
+// The wave kernel's form follows from the grid: all its waves on a segment, or,
+// with more segments than one workgroup per CU can take, one wave per head of
+// each, several workgroups per CU.  (Either form runs any plan.)  Plans have that
+// many segments where they were made for the narrow form, or where the page cap
+// asks for them; those of the latter, long segments, run narrow only if that
+// leaves no more than a quarter of the chip's waves out.
+template <int G, int D>
+void launch_wave(const DecodeArgs& a, dim3 grid, int hpw, hipStream_t s) {
+  constexpr int kWaves = WaveCfg<G, D>::kWaves;
+  const int64_t workgroups = int64_t(grid.x) * grid.y;
+  const bool capped = a.total_pages > kMaxSegPages / 2 * int64_t(grid.x);
+  if (workgroups > kChipCus && (!capped || workgroups * hpw >= kChipCus * kWaves * 3 / 4))
+    decode_wave_kernel<G, D, true><<<grid, 64 * hpw, 0, s>>>(a);
+  else
+    decode_wave_kernel<G, D, false><<<grid, 64 * kWaves, 0, s>>>(a);
+}
+
 template <int G, int D>
 void launch_segments(const DecodeArgs& a, int segments, int head_groups, int hpw,
                      hipStream_t s) {
@@ -1655,9 +1695,9 @@ void launch_segments(const DecodeArgs& a, int segments, int head_groups, int hpw
   if constexpr (D == 256 && G == 8) {
     DecodeArgs b = a;
     b.q_splits = 2;
-    decode_wave_kernel<4, D><<<dim3{grid.x, 2 * grid.y}, 64 * WaveCfg<4, D>::kWaves, 0, s>>>(b);
+    launch_wave<4, D>(b, dim3{grid.x, 2 * grid.y}, hpw, s);
   } else {
-    decode_wave_kernel<G, D><<<grid, 64 * WaveCfg<G, D>::kWaves, 0, s>>>(a);
+    launch_wave<G, D>(a, grid, hpw, s);
   }
 }
 
@@ -1852,17 +1892,6 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
     return ok();
   }
 
-  // Short requests without the per-request kernel (head_dim 64 / 256): one
-  // segment each, so that none is cut and no merge follows.
-  if (head_dim != 128 && num_segments_hint <= 0 && max_pages > 1 &&
-      max_pages <= kSmallMaxPages) {
-    cut.clear();
-    for (int i = 0; i < batch; ++i)
-      if (indptr_host[i + 1] > indptr_host[i]) cut.push_back(indptr_host[i]);
-    segs = int64_t(cut.size());
-    cut.push_back(total);
-  }
-
   // Few pages for the LDS kernel's 8-head workgroups: at two or three pages
   // each they are all start-up and cut a long request into up to 256 pieces.
   // The wave kernel on 1, 2 or 4 heads per workgroup streams longer segments;
@@ -1883,6 +1912,60 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
     hpw = group < 4 ? 2 : mean < 48 ? 4 : work <= 3 * slots ? 1 : 2;
     segs = segment_count(hpw);
     cut = cut_segments(indptr_host, batch, total, segs);
+  }
+
+  // Many requests per segment of the wave kernel: its waves would share every
+  // request and meet at its end.  The narrow form, a wave per head and segment,
+  // closes pieces without meeting; its segments are as many as the chip has waves
+  // for (at most 8 per CU, at least two pages each), or three quarters of that.  It
+  // is taken where a request has at most about kSpecParts of them, so that the
+  // merge stays one batch of loads, where they are more than the other form runs at
+  // once, and where its partials fit the allocation-free run or are no more than
+  // the other's.
+  // Measured, waves on a segment together -> narrow, us a layer:
+  //   1000 requests of 1-300 tokens, group 4, head_dim 128: 1 KV head 38.1 -> 25.9,
+  //     2 50.9 -> 42.3, 3 85.9 -> 60.5, 4 82.0 -> 75.4; 8, group 8 182 -> 161
+  //   the same, 8 KV heads, head_dim 64: group 1 81.2 -> 69.5, 4 93.0 -> 79.0,
+  //     8 133 -> 98; 64 of 200-600, group 1 20.8 -> 18.9, 4 21.7 -> 20.0
+  //   128 of 100-2000, head_dim 128, group 4: 1 KV head 22.9 -> 21.6, 4 55.0 -> 54.5
+  // Not at head_dim 256: 128 of 100-2000, 2 KV heads, group 8 80 -> 91.
+  if (hpw < kLdsHeads && num_segments_hint <= 0) {
+    const int64_t requests = batch - num_empty;
+    const int64_t waves = slots * wave_kernel_waves(group, head_dim);
+    const int64_t heads = int64_t(num_kv_heads) * q_splits;  // waves of a narrow segment
+    int64_t narrow =
+        std::min({std::max<int64_t>(1, waves / heads), total / 2, kNarrowPerCu * slots});
+    const int64_t most = kSpecParts * requests;
+    if (4 * most * heads >= 3 * waves) narrow = std::min(narrow, most);
+    const bool fits = num_segments_hint == 0 && head_dim < 256 && narrow <= most &&
+                      2 * narrow * heads > 3 * slots * hpw;
+    // Short requests of head_dim 64 / 256 (128 has its own kernel): one segment
+    // each, so that none is cut and no merge follows, in the narrow form where
+    // they fill three quarters of its waves, else where they are one round of the
+    // other form's workgroups (two for groups, whose merge costs more).
+    //   8 KV heads, 1024 of 17-32 tokens: head_dim 64, group 1 40.4 -> 22.3 us, 4
+    //   51.2 -> 24.5; head_dim 256, group 4 95 -> 69.  256 of 17-100, narrow
+    //   segments against one each: head_dim 64, group 1 17.7 and 20.2, 4 21.7 and 19.4
+    if (head_dim != 128 && max_pages > 1 && max_pages <= kSmallMaxPages &&
+        (4 * requests * heads >= 3 * waves ||
+         requests * heads <= (group == 1 ? 1 : 2) * slots * hpw || !fits)) {
+      cut.clear();
+      for (int i = 0; i < batch; ++i)
+        if (indptr_host[i + 1] > indptr_host[i]) cut.push_back(indptr_host[i]);
+      segs = int64_t(cut.size());
+      cut.push_back(total);
+    } else if (fits) {
+      const int64_t rounds = (total + kMaxSegPages * narrow - 1) / (kMaxSegPages * narrow);
+      std::vector<int64_t> cut_n = cut_segments(indptr_host, batch, total, rounds * narrow);
+      auto partials = [&](const std::vector<int64_t>& c) {
+        return kvc_decode_workspace_bytes(batch, num_qo_heads, head_dim,
+                                          most_pieces(indptr_host, batch, c));
+      };
+      if (partials(cut_n) <= std::max<int64_t>(KVC_NOALLOC_SCRATCH_BYTES, partials(cut))) {
+        segs = rounds * narrow;
+        cut = std::move(cut_n);
+      }
+    }
   }
   const int head_groups = num_kv_heads / hpw;
 

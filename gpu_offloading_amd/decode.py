@@ -136,22 +136,25 @@ class BatchDecodeWithPagedKVCacheWrapper:
         # run, so plan() never waits for the GPU.
         lib = _lib.load()
         sched = _lib.KvcDecodeSchedule()
+        ws = self._ws_args[1]
         cap = lib.kvc_decode_plan_ints(batch, max(self._segments_hint, 8 * self._num_cus))
-        for _ in range(2):
+        hint = self._segments_hint
+        while True:
             cap4 = (cap + 3) // 4 * 4
             hs = torch.empty(cap4 + 2 * batch + 1, dtype=torch.int32, pin_memory=True)
             st = lib.kvc_decode_plan(indptr_host.data_ptr(), lpl_host.data_ptr(), batch,
                                      num_qo_heads, num_kv_heads,
-                                     head_dim, page_size, self._segments_hint, self._num_cus,
+                                     head_dim, page_size, hint, self._num_cus,
                                      sched, hs.data_ptr(), cap4)
             if st == _lib.KVC_ERR_WORKSPACE and sched.plan_ints > cap4:
                 cap = sched.plan_ints
                 continue
             _lib.check("kvc_decode_plan", st)
-            break
-        ws = self._workspace.numel() * self._workspace.element_size()
-        if sched.workspace_bytes > ws:
-            _fail(f"decode workspace too small: need {sched.workspace_bytes} bytes, have {ws}")
+            if sched.workspace_bytes <= ws:
+                break
+            if hint != 0:
+                _fail(f"decode workspace too small: need {sched.workspace_bytes} bytes, have {ws}")
+            hint = -1   # the plan with fewer partials
 
         dev = self._device
         hs[cap4: cap4 + batch + 1].copy_(indptr_host)
@@ -244,16 +247,20 @@ class BatchDecodeWithPagedKVCacheWrapper:
         else:
             ptr, size = image.data_ptr(), image.numel()
         sched = _lib.KvcDecodeSchedule()
-        st = _lib.load().kvc_decode_plan(indptr_host.ctypes.data, lpl_host.ctypes.data, batch,
-                                         num_qo_heads, num_kv_heads, head_dim, page_size,
-                                         self._segments_hint, self._num_cus, sched, ptr, size)
-        if st == _lib.KVC_ERR_WORKSPACE and sched.plan_ints > size:
-            return sched
-        _lib.check("kvc_decode_plan", st)
-        ws = self._workspace.numel() * self._workspace.element_size()
-        if sched.workspace_bytes > ws:
-            _fail(f"decode workspace too small: need {sched.workspace_bytes} bytes, have {ws}")
-        return sched
+        ws = self._ws_args[1]
+        hint = self._segments_hint
+        while True:
+            st = _lib.load().kvc_decode_plan(indptr_host.ctypes.data, lpl_host.ctypes.data, batch,
+                                             num_qo_heads, num_kv_heads, head_dim, page_size,
+                                             hint, self._num_cus, sched, ptr, size)
+            if st == _lib.KVC_ERR_WORKSPACE and sched.plan_ints > size:
+                return sched
+            _lib.check("kvc_decode_plan", st)
+            if sched.workspace_bytes <= ws:
+                return sched
+            if hint != 0:
+                _fail(f"decode workspace too small: need {sched.workspace_bytes} bytes, have {ws}")
+            hint = -1   # the plan with fewer partials
 
     def _install(self, sched: _lib.KvcDecodeSchedule, plan_dev: torch.Tensor,
                  indptr_dev: torch.Tensor, lpl_dev: torch.Tensor, indices_dev: torch.Tensor,

@@ -108,8 +108,9 @@ int kvc_gather_kv(
  * kvc_decode_plan is host-only (no device access), like FlashInfer plan(),
  * which also reads a host indptr.  It cuts the batch's flattened page list
  * into num_segments segments per group of heads_per_group KV heads (by
- * default one per workgroup the GPU holds at once; num_segments_hint > 0
- * forces the count), balanced in pages plus switches between requests (at
+ * default one per workgroup the GPU holds at once, or up to 8 per CU for
+ * many requests; num_segments_hint > 0 forces the count, < 0 keeps to the
+ * former, with fewer pieces and a smaller workspace), balanced in pages plus switches between requests (at
  * most 128 pages each), and writes the plan image into plan_host:
  *   [0, 4*num_segments)          (first piece, end piece, first slot, pages)
  *   [pieces_offset, +8*pieces)   (request, first slot, end slot, partial or -1,
