@@ -1632,6 +1632,29 @@ std::vector<int64_t> cut_segments(const int32_t* indptr, int batch, int64_t tota
   return cut;
 }
 
+// Whether a request lies in more than one segment.
+bool cuts_a_request(const int32_t* indptr, int batch, const std::vector<int64_t>& cut) {
+  int b = 0;
+  for (size_t s = 1; s + 1 < cut.size(); ++s) {
+    while (b < batch && indptr[b + 1] <= cut[s]) ++b;
+    if (b < batch && indptr[b] < cut[s]) return true;
+  }
+  return false;
+}
+
+// The most leading pieces of a segment that reach the end of a request.
+int32_t leading_ends(const int32_t* indptr, int batch, const std::vector<int64_t>& cut) {
+  int32_t most = 0;
+  int b = 0;
+  for (size_t s = 0; s + 1 < cut.size(); ++s) {
+    while (b < batch && indptr[b + 1] <= cut[s]) ++b;
+    int32_t ends = 0;
+    for (int i = b; i < batch && indptr[i + 1] <= cut[s + 1]; ++i) ends += indptr[i + 1] > indptr[i];
+    most = std::max(most, ends);
+  }
+  return most;
+}
+
 // The most segments that one request lies in.
 int32_t most_pieces(const int32_t* indptr, int batch, const std::vector<int64_t>& cut) {
   int64_t most = 1;
@@ -1824,6 +1847,11 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
     }
     return std::min<int64_t>(n, total);
   };
+  auto fine_segments = [&]() -> int64_t {
+    const int64_t round = (slots * (group == 8 ? 4 : 8) + num_kv_heads - 1) / num_kv_heads;
+    const int64_t at_least = (total + kMaxSegPages - 1) / kMaxSegPages;
+    return std::min((std::max(round, at_least) + round - 1) / round * round, total);
+  };
   int64_t segs = segment_count(hpw);
   KVC_REQUIRE(segs <= (int64_t(1) << 30), KVC_ERR_INVALID_ARG, "too many segments");
 
@@ -1836,16 +1864,14 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
   int64_t max_pages = 0;
   for (int b = 0; b < batch; ++b)
     max_pages = std::max<int64_t>(max_pages, indptr_host[b + 1] - indptr_host[b]);
-  // (Where the wave kernel would stream the batch, a request of two pages or
-  // more is taken as cut: per-request workgroups are also its best schedule.)
-  bool splits = !lds && max_pages > 1;
-  for (int64_t s = 1, bb = 0; s < segs && !splits; ++s) {
-    const int64_t g = cut[size_t(s)];  // first page of segment s
-    while (bb < batch && indptr_host[bb + 1] <= g) ++bb;
-    splits = bb < batch && indptr_host[bb] < g;  // pages g-1 and g in request bb
-  }
+  // Layouts without the LDS kernel are cut here as finely as eight workgroups per
+  // CU (four for groups of 8) would be: that takes nearly every batch of requests
+  // of two pages and more but those that line up with the segments, many of a
+  // length (1024 of 31 tokens, 4 KV heads, group 4: 60 us this way, 19.5 in the
+  // wave kernel's narrow form).
   if (num_segments_hint <= 0 && head_dim == 128 && total > 0 && max_pages <= kSmallMaxPages &&
-      splits) {
+      cuts_a_request(indptr_host, batch,
+                     lds ? cut : cut_segments(indptr_host, batch, total, fine_segments()))) {
     const int64_t need = kvc_decode_plan_ints(batch, batch);
     sched->batch = batch;
     sched->num_qo_heads = num_qo_heads;
@@ -1908,7 +1934,11 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
   //     8 x 72  14.7 -> 16.2 / 15.4 / 14.8     20 x 37   16.6 -> 19.2 / 17.9 / 17.4
   const int64_t work = total * (num_kv_heads / kLdsHeads);  // pages of 8 heads
   const int64_t mean = total / std::max(1, batch - num_empty);  // pages per request
-  if (lds && num_segments_hint <= 0 && work <= 12 * slots && mean >= (group == 4 ? 16 : 96)) {
+  // Batches for which the LDS kernel cannot append keep its plan, and with it which
+  // calls take the append and which rows (40 requests of 3 tokens + 30 of 1590: 46
+  // us with the append's launch, 42 here).
+  if (lds && num_segments_hint <= 0 && work <= 12 * slots && mean >= (group == 4 ? 16 : 96) &&
+      leading_ends(indptr_host, batch, cut) <= kNewMax) {
     hpw = group < 4 ? 2 : mean < 48 ? 4 : work <= 3 * slots ? 1 : 2;
     segs = segment_count(hpw);
     cut = cut_segments(indptr_host, batch, total, segs);
