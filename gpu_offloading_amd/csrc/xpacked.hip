@@ -39,12 +39,24 @@ namespace {
 
 constexpr int kThreads = 256;
 // Waves per v2 workgroup.  164 registers let a CU hold three 4-wave workgroups or
-// one of 8 waves.  A grid of many rounds per CU reads faster through the latter
-// (64 sequences of 512-4096, 32 heads, 16384 workgroups: 355 us against 367),
+// one of 8 waves.  A grid of many rounds per CU reads faster through the latter,
 // fewer reads in flight each of neighbouring pages; a few rounds want the
-// overlap of several workgroups (6 of 16400-19000, 4 KV heads, 912: 48 against 53).
+// overlap of several workgroups, and fewer KV heads, whose pages have shorter runs
+// to read side by side, for longer.  By the workgroups launched (max_seq_len's
+// partitions, present or not: the host does not know the lengths), bf16, 4 waves
+// -> 8, us:
+//   32 KV heads:  1792 59.3 -> 61.4   4096 122 -> 117, 109 -> 107   5120 172 -> 165
+//     8192 211 -> 201   16384 412 -> 396         16:  4096 118 -> 115, 153 -> 153
+//   8 or 4 KV heads:  912 48 -> 53   4096 134 -> 137, 118 -> 125   4608 160 -> 170
+//     6144 202 -> 206   8192 256 -> 257, 263 -> 267   9216 260 -> 259, 363 -> 351
 constexpr int kV2Waves = 4, kV2WavesMany = 8;
-constexpr int64_t kManyWorkgroups = 4096;
+constexpr int64_t many_workgroups(int kv_heads) { return kv_heads >= 16 ? 4096 : 8192; }
+// Waves per v1 workgroup, which has the whole sequence: 8, or 4 where most of 8
+// would have a page pair or none.  4 -> 8, us: 64 sequences, 32 heads, of 10-30
+// tokens 21.3 -> 29.3, 100-200 38.8 -> 42.6, 200-400 62.7 -> 63.4, 300-600 88.9 ->
+// 84.5; 8 of 1000-2000, 8 KV heads, group 4 32.2 -> 28.2.
+constexpr int kV1Waves = 8, kV1WavesShort = 4;
+constexpr int kV1Short = 512;  // tokens
 constexpr int kBlock = 16;    // tokens per block
 constexpr int kD = 128;       // head size
 constexpr int kX = 8;         // elements per 16-byte chunk
@@ -435,12 +447,14 @@ __global__ __launch_bounds__(kRedThreads) void xpacked_reduce_kernel(XDecodeArgs
 template <int G, bool kBf16>
 void launch_decode(const XDecodeArgs& a, bool v1, int parts, int hkv, int seqs, hipStream_t s) {
   if (v1) {
-    // 8 waves: a workgroup has the whole sequence (4 sequences of 300-2000, 8 KV
-    // heads, group 4: 20 us, with 4 waves 23; 32 of 300-900, 32 heads: 59 and 64).
-    xpacked_decode_kernel<G, kBf16, true, 8><<<dim3(hkv, seqs, 1), 64 * 8, 0, s>>>(a);
+    const dim3 grid(hkv, seqs, 1);
+    if (parts * kPart <= kV1Short)
+      xpacked_decode_kernel<G, kBf16, true, kV1WavesShort><<<grid, 64 * kV1WavesShort, 0, s>>>(a);
+    else
+      xpacked_decode_kernel<G, kBf16, true, kV1Waves><<<grid, 64 * kV1Waves, 0, s>>>(a);
   } else {
     const dim3 grid(hkv, seqs, parts);
-    if (int64_t(hkv) * seqs * parts >= kManyWorkgroups)
+    if (int64_t(hkv) * seqs * parts >= many_workgroups(hkv))
       xpacked_decode_kernel<G, kBf16, false, kV2WavesMany><<<grid, 64 * kV2WavesMany, 0, s>>>(a);
     else
       xpacked_decode_kernel<G, kBf16, false, kV2Waves><<<grid, 64 * kV2Waves, 0, s>>>(a);

@@ -20,8 +20,9 @@ pytestmark = pytest.mark.gpu
     ("fp16", 1, 3, False), ("bf16", 4, 2, False), ("fp16", 8, 1, False)])
 def test_page_pairs_and_missing_pages(gpu, dt, group, hkv, many):
     lens = [0, 1, 15, 16, 17, 31, 32, 33, 129, 255, 257, 511, 512, 513, 545, 1100]
-    # v2 runs 8 waves from 4096 (KV head, sequence, partition) workgroups on
-    max_len = 512 * (4096 // (hkv * len(lens))) if many else 1100
+    # v2 runs 8 waves from 4096 (KV head, sequence, partition) workgroups on, with
+    # fewer than 16 KV heads from 8192
+    max_len = 512 * ((4096 if hkv >= 16 else 8192) // (hkv * len(lens))) if many else 1100
     q, kc, vc, bt = _attn_case(lens, hkv * group, hkv, dt, 90 + group, gpu)
     hidden = [(9, 3, -1), (10, 0, kc.shape[0]), (10, 1, -1), (13, 31, -1), (13, 32, -1),
               (14, 34, kc.shape[0] + 3)] + [(15, p, -1) for p in range(2, 20)]
@@ -49,3 +50,21 @@ def test_page_pairs_and_missing_pages(gpu, dt, group, hkv, many):
     out2, *_ = _run_v2(q, kc, vc, bt, lens, hkv, scale, gpu, max_seq_len=max_len)
     for out in (out1, out2):
         assert_attn_close(out.float().cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("dt,group,hkv", [("fp16", 1, 8), ("bf16", 4, 2), ("fp16", 8, 1)])
+@pytest.mark.parametrize("longest", [512, 513])   # v1: 4 waves, 8 from the second partition on
+def test_v1_of_short_sequences(gpu, dt, group, hkv, longest):
+    lens = [0, 1, 16, 17, 33, 100, 128, 129, 160, 255, 257, longest]
+    q, kc, vc, bt = _attn_case(lens, hkv * group, hkv, dt, 130 + group, gpu)
+    for b, n in enumerate(lens):
+        if n % 16:
+            kc[bt[b, n // 16], :, :, n % 16:] = float("nan")
+            vc[bt[b, n // 16], :, :, n % 16:] = float("nan")
+    ref, *_ = orc.paged_attention_xpacked(u16(q), u16(kc), u16(vc), bt, np.array(lens), 0.08,
+                                          dtype=dt)
+    out = torch.empty_like(q)
+    ops.paged_attention_v1(out, q, kc, vc, hkv, 0.08, torch.from_numpy(bt).to(gpu),
+                           torch.tensor(lens, dtype=torch.int32, device=gpu), 16, longest,
+                           None, "auto", 1.0, 1.0)
+    assert_attn_close(out.float().cpu().numpy(), ref)
