@@ -1920,24 +1920,29 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
 
   // Few pages for the LDS kernel's 8-head workgroups: at two or three pages
   // each they are all start-up and cut a long request into up to 256 pieces.
-  // The wave kernel on 1, 2 or 4 heads per workgroup streams longer segments;
-  // the shorter the requests, the more heads, so that a workgroup's waves do
-  // not meet at a piece's end too often.  Measured with 8 KV heads, one layer
-  // with its append, LDS kernel -> 1 / 2 / 4 heads, in us:
-  //   group 4, requests x pages:  1 x 256  25.3 -> 12.9 / 13.8 / 17.8
-  //     8 x 68  18.3 -> 15.0 / 15.5 / 16.7     16 x 110  30.9 -> 30.3 / 28.9 / 28.3
-  //     20 x 37 19.9 -> 19.2 / 18.6 / 18.6     60 x 27   28.8 -> 30.2 / 27.9 / 27.6
-  //     12 x 14 12.5 -> 13.2 / 12.5 / 12.4     32 x 128  51.1 -> 55.0 / 51.7 / 50.7
-  //   (wave kernel with 12 waves; with the 8 it has now 8 x 68 takes 1 us less)
-  //   groups 1, 2 (the LDS kernel's arithmetic is a quarter or half of that):
-  //     2 x 138 18.3 -> 13.3 / 12.9 / 14.9     4 x 131   16.6 -> 16.4 / 15.5 / 16.0
-  //     8 x 72  14.7 -> 16.2 / 15.4 / 14.8     20 x 37   16.6 -> 19.2 / 17.9 / 17.4
+  // The wave kernel streams longer segments on 1, 2 or 4 heads per workgroup, of
+  // which the shorter the requests, the more (in its narrow form, below, they are
+  // alike).  Measured with 8 KV heads, one layer with its append, LDS kernel ->
+  // 1 / 2 / 4 heads, in us:
+  //   group 4, requests x pages:  1 x 256  26.0 -> 12.8 / 13.9 / 18.1
+  //     2 x 500 28.3 -> 19.3 / 19.8 / 21.3     4 x 40    13.1 -> 11.1 / 11.2 / 13.0
+  //     8 x 68  20.1 -> 14.4 / 14.0 / 14.7     16 x 110  29.1 -> 26.0 / 25.9 / 25.9
+  //     20 x 37 19.7 -> 17.4 / 17.3 / 17.4     60 x 27   29.4 -> 26.4 / 26.6 / 26.4
+  //     150 x 20 44.2 -> 42.6 / 43.3 / 42.6    12 x 250  41.6 -> 37.9 / 38.0 / 38.2
+  //   groups 1, 2 (the LDS kernel's arithmetic is a quarter or half of that; group
+  //   1's figures):
+  //     2 x 138 16.7 -> 11.7 / 11.8 / 13.0     4 x 131   16.2 -> 13.7 / 13.2 / 13.8
+  //     8 x 72  15.0 -> 14.1 / 13.4 / 13.6     1 x 2900  48.0 -> 39.1 / 38.0 / 40.2
+  //     30 x 50 23.2 -> 22.7 / 22.6 / 22.7     30 x 100  37.1 -> 36.3 / 36.5 / 36.3
+  //     20 x 37 15.4 -> 15.8 / 15.7 / 15.6
+  //   above 12 pages per CU and KV head group the LDS kernel has long segments, too
+  //   (64 requests of 512-4096 tokens: at 6.2 of 7.0 TB/s)
   const int64_t work = total * (num_kv_heads / kLdsHeads);  // pages of 8 heads
   const int64_t mean = total / std::max(1, batch - num_empty);  // pages per request
   // Batches for which the LDS kernel cannot append keep its plan, and with it which
   // calls take the append and which rows (40 requests of 3 tokens + 30 of 1590: 46
   // us with the append's launch, 42 here).
-  if (lds && num_segments_hint <= 0 && work <= 12 * slots && mean >= (group == 4 ? 16 : 96) &&
+  if (lds && num_segments_hint <= 0 && work <= 12 * slots && mean >= (group == 4 ? 16 : 48) &&
       leading_ends(indptr_host, batch, cut) <= kNewMax) {
     hpw = group < 4 ? 2 : mean < 48 ? 4 : work <= 3 * slots ? 1 : 2;
     segs = segment_count(hpw);
