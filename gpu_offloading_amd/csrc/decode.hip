@@ -1550,7 +1550,8 @@ __global__ __launch_bounds__(64 * kManyWaves) void decode_merge_many_kernel(Merg
   for (int e = 0; e < EPL; ++e) s_acc[wave][lane * EPL + e] = acc[e];
   __syncthreads();
   S = wave_sum(S);
-  const float inv = S > 0.f ? 1.f / S : 0.f;  // no pages, or none present: 0 and -inf
+  const bool none = mx == -INFINITY;  // no pages, or none present: 0 and -inf
+  const float inv = none ? 0.f : 1.f / S;
   uint16_t* out = a.out + int64_t(b) * a.out_stride + int64_t(hq) * D;
   for (int d = threadIdx.x; d < D; d += 64 * kManyWaves) {
     float o = 0.f;
@@ -1559,7 +1560,7 @@ __global__ __launch_bounds__(64 * kManyWaves) void decode_merge_many_kernel(Merg
     out[d] = f32_to_bf16(o * inv);
   }
   if (a.lse && threadIdx.x == 0)
-    a.lse[int64_t(b) * a.num_kv_heads * G + hq] = S > 0.f ? (mx + fast_log2(S)) * kLn2 : -INFINITY;
+    a.lse[int64_t(b) * a.num_kv_heads * G + hq] = none ? -INFINITY : (mx + fast_log2(S)) * kLn2;
 }
 
 template <int D>
