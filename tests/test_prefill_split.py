@@ -177,3 +177,14 @@ def test_without_workspace_the_whole_units_run(gpu):
                   _lib.current_stream_handle(torch.device(gpu)))
         torch.cuda.synchronize()
         check(out, lse)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kv_len,group,parts", [(30000, 8, 117), (17100, 4, 67), (20000, 2, 78)])
+def test_merge_of_more_partials_than_lanes(gpu, kv_len, group, parts):
+    """One chunk over a long history: the merge's maximum takes a second pass over
+    the partials, its fold many, with a remainder of a batch of eight."""
+    w, *_ = _check(gpu, [40], [kv_len], group, 1, 90 + group, True)
+    s = w._sched.split
+    merges = w._plan_dev[s.merges_offset:s.merges_offset + 8 * s.num_merges].cpu().view(-1, 8)
+    assert int(merges[:, 4].max()) == parts
