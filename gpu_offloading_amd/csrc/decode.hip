@@ -190,15 +190,11 @@ __device__ __forceinline__ void write_piece(const DecodeArgs& a, const int4& pc,
   const int hq = h * group + g;
   if (pc.w < 0) {
     uint16_t* dst = a.out + int64_t(b) * a.out_stride + int64_t(hq) * D + d0;
-    if constexpr (NDIM % 2 == 0) {
+    static_assert(NDIM % 2 == 0, "dims are stored in pairs");
 #pragma unroll
-      for (int e = 0; e < NDIM; e += 2)
-        *reinterpret_cast<uint32_t*>(dst + e) =
-            uint32_t(f32_to_bf16(o[e])) | (uint32_t(f32_to_bf16(o[e + 1])) << 16);
-    } else {
-#pragma unroll
-      for (int e = 0; e < NDIM; ++e) dst[e] = f32_to_bf16(o[e]);
-    }
+    for (int e = 0; e < NDIM; e += 2)
+      *reinterpret_cast<uint32_t*>(dst + e) =
+          uint32_t(f32_to_bf16(o[e])) | (uint32_t(f32_to_bf16(o[e + 1])) << 16);
     if (a.lse && lse_lane)
       a.lse[int64_t(b) * a.num_kv_heads * group + hq] = lse2 * kLn2;
   } else {
@@ -792,9 +788,11 @@ __global__ __launch_bounds__(64 * kSmallWaves) void decode_small_kernel(DecodeAr
 // small: K and V go from memory into registers, nothing is staged in LDS, and
 // no barrier sits in the page loop.  A workgroup's waves are its KV heads times
 // TS page shares: wave (head, ts) streams units ts, ts + TS, ... of the
-// segment (a unit is one page, at head_dim 64 below group 8 two).  One unit is in flight per
-// wave while another is consumed -- K's registers are refilled as soon as q.k
-// has read them, V's after p.v -- and 8 to 16 waves per CU hide the latency.
+// segment (a unit is one page, at head_dim 64 below group 8 two); in the narrow
+// form, for many requests per segment, a workgroup is its heads' waves alone, each
+// on all units, and several workgroups share a CU.  One unit is in flight per wave
+// while another is consumed -- K's registers are refilled as soon as q.k has read
+// them, V's after p.v -- 64 KB and more a CU with the waves of WaveCfg.
 // Every K and V load of the wave reads whole token rows (four rows of 256 B at
 // head_dim 128), which the layouts of the 4x4 matrix instructions allow:
 //   q.k : v_mfma_f32_4x4x4_16b_bf16, block b = 16-byte chunk b of a row, rows =
@@ -816,11 +814,11 @@ __global__ __launch_bounds__(64 * kSmallWaves) void decode_small_kernel(DecodeAr
 //
 // One layer with its append (start: the kernel it replaces with the merge of
 // its time), us:
-//   32 requests of 500-3001 tokens, 8 KV heads, group 8, head_dim 64: 63.8 -> 32.5
-//   64 of 512-4096, group 8, head_dim 128: 133 -> 101 (5.6 TB/s)
+//   32 requests of 500-3001 tokens, 8 KV heads, group 8, head_dim 64: 63.8 -> 30.6
+//   64 of 512-4096, 8 KV heads, group 8, head_dim 128: 149 -> 110 (5.6 TB/s)
 //   64 of 512-4096, one KV head, group 4, head_dim 128: 35.6 -> 20.1
-//   32 of 500-3000, 8 KV heads, head_dim 256, group 4: 93 -> 80 (5.7 TB/s)
-//   32 of 500-3000, 16 KV heads, head_dim 64, group 1: 47.9 -> 44.8
+//   32 of 500-3000, 8 KV heads, head_dim 256, group 4: 100 -> 87 (5.5 TB/s)
+//   64 of 512-4096, 16 KV heads, head_dim 64, group 1: 109 -> 100
 // ---------------------------------------------------------------------------
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
@@ -960,7 +958,9 @@ __global__ __launch_bounds__((64 * (kNarrow ? kMaxWaveHeads : WaveCfg<G, D>::kWa
   const int group = G * a.q_splits;  // query heads of a KV head
   const int4 segment = scalar_int4(a.segments, blockIdx.x);
   int k = segment.x;
-  const int k_end = segment.y, g0 = segment.z, n = segment.w;
+  const int k_end = segment.y;
+  int g0, n;
+  segment_span(segment, g0, n);
   if (k >= k_end) return;  // uniform over the workgroup
 
   // Lane roles.  K (and q.k): row of four consecutive tokens l % 4, 16-byte
@@ -990,14 +990,17 @@ __global__ __launch_bounds__((64 * (kNarrow ? kMaxWaveHeads : WaveCfg<G, D>::kWa
   const int64_t block_bytes = a.block_stride * 2;
 
   // This wave's units of PU consecutive pages: unit ts, ts + TS, ... of the
-  // segment; the pages' ids one per lane.
+  // segment; the pages' ids one per lane (a wave that shares the segment has at most
+  // half of its pages).
   const int nw = n > PU * ts ? (n - PU * ts + PU * TS - 1) / (PU * TS) : 0;
   auto page_slot = [&](int j, int x) { return g0 + PU * (ts + TS * j) + x; };
-  int32_t idr[kIdRegs];
+  constexpr int IR = kNarrow ? kIdRegs : kIdRegs / 2;
+  static_assert(kNarrow || W >= 2 * kMaxWaveHeads, "two waves at least share a segment");
+  int32_t idr[IR];
   {
     const int64_t last = a.num_indices - 1;
 #pragma unroll
-    for (int i = 0; i < kIdRegs; ++i) {
+    for (int i = 0; i < IR; ++i) {
       idr[i] = -1;
       if (64 * i < PU * nw) {
         const int j = lane + 64 * i;
@@ -1010,7 +1013,7 @@ __global__ __launch_bounds__((64 * (kNarrow ? kMaxWaveHeads : WaveCfg<G, D>::kWa
   auto id_at = [&](int j) __attribute__((always_inline)) {
     int32_t v = __builtin_amdgcn_readlane(idr[0], j & 63);
 #pragma unroll
-    for (int i = 1; i < kIdRegs; ++i) {
+    for (int i = 1; i < IR; ++i) {
       const int32_t x = __builtin_amdgcn_readlane(idr[i], j & 63);
       v = (j >> 6) == i ? x : v;
     }
@@ -1677,7 +1680,11 @@ bool lds_layout(int group, int head_dim, int num_kv_heads) {
 
 // KV heads per workgroup of the wave kernel: its waves are split between heads
 // and pages.  More heads read longer runs of each token row, fewer leave longer
-// segments and so fewer pieces to merge.
+// segments and so fewer pieces to merge.  Heads in twos (6, 10, 14) are taken two
+// at a time where rows are short or long: 6 heads, 1 -> 2 per workgroup, us: 8
+// requests of 300-2000 tokens, head_dim 64, groups 1 and 4 14.6 -> 13.9, 14.3 -> 13.0
+// (narrow form, 32 of 500-3000: 24.6 -> 24.9, 25.0 -> 26.0); 32 of 500-3000, head_dim
+// 256 63.2 -> 59.9, 61.7 -> 59.6; at 128 33.5 and 33.6, 36.5 and 36.4.
 int wave_heads(int head_dim, int num_kv_heads) {
   if (num_kv_heads % 4 == 0) return 4;
   return num_kv_heads == 2 || (head_dim != 128 && num_kv_heads % 2 == 0) ? 2 : 1;
