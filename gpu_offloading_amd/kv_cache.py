@@ -652,8 +652,8 @@ class PagedKVCache:
         if (s is None or self._step_dev is None or self._step_slots is None
                 or w._plan_dev.data_ptr() != self._step_dev.data_ptr()):
             return ()   # no decode step set up (or a mixed step's plan is current)
-        # Without the fused append, append_and_decode's separate append reads
-        # the step's slot tensor, a new allocation every step.
+        # Without the fused append, append_and_decode may make a separate append,
+        # which reads the step's slot tensor (a new one when a step outgrows it).
         slots = 0 if w.fused_append_supported else self._step_slots.data_ptr()
         return (self._step_dev.data_ptr(), w._indices.data_ptr(), w._num_indices, slots,
                 s.batch, s.small_batch, s.num_segments,
