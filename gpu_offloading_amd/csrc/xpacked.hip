@@ -49,12 +49,21 @@ constexpr int kThreads = 256;
 //     8192 211 -> 201   16384 412 -> 396         16:  4096 118 -> 115, 153 -> 153
 //   8 or 4 KV heads:  912 48 -> 53   4096 134 -> 137, 118 -> 125   4608 160 -> 170
 //     6144 202 -> 206   8192 256 -> 257, 263 -> 267   9216 260 -> 259, 363 -> 351
+// A grid of at most one workgroup per CU has nothing to overlap and shares a
+// partition's 16 page pairs between 8, too: 8 to 256 workgroups 2-12% faster (a
+// sequence of 100-200, 32 heads 8.7 -> 8.2, of 1500-2000, 8 heads, group 4 13.0 ->
+// 11.7), 288 to 576 5-10% slower.
 constexpr int kV2Waves = 4, kV2WavesMany = 8;
-constexpr int64_t many_workgroups(int kv_heads) { return kv_heads >= 16 ? 4096 : 8192; }
-// Waves per v1 workgroup, which has the whole sequence: 8, or 4 where most of 8
-// would have a page pair or none.  4 -> 8, us: 64 sequences, 32 heads, of 10-30
-// tokens 21.3 -> 29.3, 100-200 38.8 -> 42.6, 200-400 62.7 -> 63.4, 300-600 88.9 ->
-// 84.5; 8 of 1000-2000, 8 KV heads, group 4 32.2 -> 28.2.
+constexpr int64_t kChipCus = 256;
+constexpr bool v2_many_waves(int64_t workgroups, int kv_heads) {
+  return workgroups <= kChipCus || workgroups >= (kv_heads >= 16 ? 4096 : 8192);
+}
+// Waves per v1 workgroup, which has the whole sequence: 8, or 4 where there are
+// several workgroups per CU and most of 8 waves would have a page pair or none.  4
+// -> 8, us: 64 sequences, 32 heads, of 20-60 tokens 18.5 -> 26.1, 100-200 32.8 ->
+// 36.1, 300-480 73.9 -> 72.8; 32 of 300-480, 16 heads 21.4 -> 22.6; one of 100-200,
+// 32 heads 6.8 -> 6.2, of 300-480 7.9 -> 6.9; 8 of 1000-2000, 8 heads, group 4 32.2
+// -> 28.2.
 constexpr int kV1Waves = 8, kV1WavesShort = 4;
 constexpr int kV1Short = 512;  // tokens
 constexpr int kBlock = 16;    // tokens per block
@@ -448,13 +457,13 @@ template <int G, bool kBf16>
 void launch_decode(const XDecodeArgs& a, bool v1, int parts, int hkv, int seqs, hipStream_t s) {
   if (v1) {
     const dim3 grid(hkv, seqs, 1);
-    if (parts * kPart <= kV1Short)
+    if (parts * kPart <= kV1Short && int64_t(hkv) * seqs > kChipCus)
       xpacked_decode_kernel<G, kBf16, true, kV1WavesShort><<<grid, 64 * kV1WavesShort, 0, s>>>(a);
     else
       xpacked_decode_kernel<G, kBf16, true, kV1Waves><<<grid, 64 * kV1Waves, 0, s>>>(a);
   } else {
     const dim3 grid(hkv, seqs, parts);
-    if (int64_t(hkv) * seqs * parts >= many_workgroups(hkv))
+    if (v2_many_waves(int64_t(hkv) * seqs * parts, hkv))
       xpacked_decode_kernel<G, kBf16, false, kV2WavesMany><<<grid, 64 * kV2WavesMany, 0, s>>>(a);
     else
       xpacked_decode_kernel<G, kBf16, false, kV2Waves><<<grid, 64 * kV2Waves, 0, s>>>(a);

@@ -17,11 +17,12 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dt,group,hkv,many", [
     ("fp16", 1, 32, True), ("bf16", 2, 16, True), ("bf16", 8, 4, True),
-    ("fp16", 1, 3, False), ("bf16", 4, 2, False), ("fp16", 8, 1, False)])
+    ("fp16", 1, 3, False), ("bf16", 4, 2, False), ("fp16", 8, 1, False),
+    ("fp16", 1, 8, False), ("bf16", 4, 6, False), ("bf16", 8, 6, False)])
 def test_page_pairs_and_missing_pages(gpu, dt, group, hkv, many):
     lens = [0, 1, 15, 16, 17, 31, 32, 33, 129, 255, 257, 511, 512, 513, 545, 1100]
     # v2 runs 8 waves from 4096 (KV head, sequence, partition) workgroups on, with
-    # fewer than 16 KV heads from 8192
+    # fewer than 16 KV heads from 8192, and up to 256; here 48, 96, 144 and 288, 384
     max_len = 512 * ((4096 if hkv >= 16 else 8192) // (hkv * len(lens))) if many else 1100
     q, kc, vc, bt = _attn_case(lens, hkv * group, hkv, dt, 90 + group, gpu)
     hidden = [(9, 3, -1), (10, 0, kc.shape[0]), (10, 1, -1), (13, 31, -1), (13, 32, -1),
@@ -53,9 +54,11 @@ def test_page_pairs_and_missing_pages(gpu, dt, group, hkv, many):
 
 
 @pytest.mark.parametrize("dt,group,hkv", [("fp16", 1, 8), ("bf16", 4, 2), ("fp16", 8, 1)])
-@pytest.mark.parametrize("longest", [512, 513])   # v1: 4 waves, 8 from the second partition on
-def test_v1_of_short_sequences(gpu, dt, group, hkv, longest):
-    lens = [0, 1, 16, 17, 33, 100, 128, 129, 160, 255, 257, longest]
+@pytest.mark.parametrize("longest", [512, 513])
+@pytest.mark.parametrize("times", [1, 26])
+def test_v1_of_short_sequences(gpu, dt, group, hkv, longest, times):
+    # v1: 4 waves up to 512 tokens and from 257 workgroups (here 12 to 312 a KV head)
+    lens = [0, 1, 16, 17, 33, 100, 128, 129, 160, 255, 257, longest] * times
     q, kc, vc, bt = _attn_case(lens, hkv * group, hkv, dt, 130 + group, gpu)
     for b, n in enumerate(lens):
         if n % 16:
