@@ -1982,6 +1982,10 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
     if (4 * most * heads >= 3 * waves) narrow = std::min(narrow, most);
     const bool fits = num_segments_hint == 0 && head_dim < 256 && narrow <= most &&
                       2 * narrow * heads > 3 * slots * hpw;
+    auto partials = [&](const std::vector<int64_t>& c) {
+      return kvc_decode_workspace_bytes(batch, num_qo_heads, head_dim,
+                                        most_pieces(indptr_host, batch, c));
+    };
     // Short requests of head_dim 64 / 256 (128 has its own kernel): one segment
     // each, so that none is cut and no merge follows, in the narrow form where
     // they fill three quarters of its waves, else where they are one round of the
@@ -1989,7 +1993,22 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
     //   8 KV heads, 1024 of 17-32 tokens: head_dim 64, group 1 40.4 -> 22.3 us, 4
     //   51.2 -> 24.5; head_dim 256, group 4 95 -> 69.  256 of 17-100, narrow
     //   segments against one each: head_dim 64, group 1 17.7 and 20.2, 4 21.7 and 19.4
+    // Not where a workgroup is on its request's pages longer than the segments on
+    // theirs and a merge: CUs are idle meanwhile.  A page of one head is about 0.12
+    // us at head_dim 64, 0.35 at 256.  One segment each -> cut, 8 requests (or
+    // 64), 4 KV heads, us by pages of a request:
+    //   head_dim 64, group 1    5  7.5 -> 7.9    7  8.7 -> 8.0   16 12.6 -> 8.8
+    //     group 4               5  8.1 -> 8.3    7  8.9 -> 8.5   16 12.1 -> 9.1
+    //   head_dim 256, group 1   2  8.5 -> 10.0   4 12.0 -> 10.2  16 28.0 -> 11.1
+    //     group 4               2 10.8 -> 10.4   4 14.0 -> 10.7  16 28.1 -> 11.8
+    //     group 1, 64 requests  5 13.7 -> 14.0   8 18.0 -> 16.3  16 29.7 -> 21.5
+    // With no partials to be had (a negative hint), or more than the allocation-free
+    // run has, the requests stay whole.
+    const int64_t longest = segs > 0 ? (total + segs - 1) / segs : 0;
+    const int64_t alone = head_dim == 256 ? 6 : group == 8 ? 8 : 16;  // pages of a head
     if (head_dim != 128 && max_pages > 1 && max_pages <= kSmallMaxPages &&
+        (num_segments_hint < 0 || (max_pages - 2 * longest) * hpw <= alone ||
+         partials(cut) > KVC_NOALLOC_SCRATCH_BYTES) &&
         (4 * requests * heads >= 3 * waves ||
          requests * heads <= (group == 1 ? 1 : 2) * slots * hpw || !fits)) {
       cut.clear();
@@ -2000,10 +2019,6 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
     } else if (fits) {
       const int64_t rounds = (total + kMaxSegPages * narrow - 1) / (kMaxSegPages * narrow);
       std::vector<int64_t> cut_n = cut_segments(indptr_host, batch, total, rounds * narrow);
-      auto partials = [&](const std::vector<int64_t>& c) {
-        return kvc_decode_workspace_bytes(batch, num_qo_heads, head_dim,
-                                          most_pieces(indptr_host, batch, c));
-      };
       if (partials(cut_n) <= std::max<int64_t>(KVC_NOALLOC_SCRATCH_BYTES, partials(cut))) {
         segs = rounds * narrow;
         cut = std::move(cut_n);
