@@ -1875,7 +1875,7 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
   // Layouts without the LDS kernel are cut here as finely as eight workgroups per
   // CU (four for groups of 8) would be: that takes nearly every batch of requests
   // of two pages and more but those that line up with the segments, many of a
-  // length (1024 of 31 tokens, 4 KV heads, group 4: 60 us this way, 19.5 in the
+  // length (1024 of 26 tokens, 4 KV heads, group 4: 59 us this way, 18.6 in the
   // wave kernel's narrow form).
   if (num_segments_hint <= 0 && head_dim == 128 && total > 0 && max_pages <= kSmallMaxPages &&
       cuts_a_request(indptr_host, batch,
@@ -1986,31 +1986,47 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
       return kvc_decode_workspace_bytes(batch, num_qo_heads, head_dim,
                                         most_pieces(indptr_host, batch, c));
     };
-    // Short requests of head_dim 64 / 256 (128 has its own kernel): one segment
-    // each, so that none is cut and no merge follows, in the narrow form where
-    // they fill three quarters of its waves, else where they are one round of the
-    // other form's workgroups (two for groups, whose merge costs more).
+    // Short requests: one segment each, so that none is cut and no merge follows.
+    // At head_dim 128 these are the many, alike in length, that the kernel above
+    // leaves; the narrow form's balanced segments would cut them all but for a few
+    // head counts (group 4, 6 KV heads: 342 of 26 tokens 20.7 -> 10.9 us, 1368 of 180
+    // 170 -> 146; group 8, 1 head, 1024 of 66 23.3 -> 13.9; 4 heads, where 1024 of
+    // 66 are not cut, 37.8 and 40.8).
+    // At head_dim 64 and 256, in the narrow form where they fill three quarters of
+    // its waves, else where they are one round of the other form's workgroups (two
+    // for groups, whose merge costs more).
     //   8 KV heads, 1024 of 17-32 tokens: head_dim 64, group 1 40.4 -> 22.3 us, 4
     //   51.2 -> 24.5; head_dim 256, group 4 95 -> 69.  256 of 17-100, narrow
     //   segments against one each: head_dim 64, group 1 17.7 and 20.2, 4 21.7 and 19.4
-    // Not where a workgroup is on its request's pages longer than the segments on
-    // theirs and a merge: CUs are idle meanwhile.  A page of one head is about 0.12
-    // us at head_dim 64, 0.35 at 256.  One segment each -> cut, 8 requests (or
-    // 64), 4 KV heads, us by pages of a request:
-    //   head_dim 64, group 1    5  7.5 -> 7.9    7  8.7 -> 8.0   16 12.6 -> 8.8
-    //     group 4               5  8.1 -> 8.3    7  8.9 -> 8.5   16 12.1 -> 9.1
-    //   head_dim 256, group 1   2  8.5 -> 10.0   4 12.0 -> 10.2  16 28.0 -> 11.1
-    //     group 4               2 10.8 -> 10.4   4 14.0 -> 10.7  16 28.1 -> 11.8
-    //     group 1, 64 requests  5 13.7 -> 14.0   8 18.0 -> 16.3  16 29.7 -> 21.5
-    // With no partials to be had (a negative hint), or more than the allocation-free
-    // run has, the requests stay whole.
+    // While CUs are left over, with fewer heads per workgroup (few), so that more
+    // waves share a request's pages.  8 requests, 4 KV heads, us by pages of a
+    // request, 4 heads per workgroup -> 1 (and cut, 4 heads per workgroup):
+    //   head_dim 64, group 1    3  6.6 -> 7.2 (7.9)    7  8.7 -> 7.3 (8.0)
+    //                          16 12.6 -> 8.7 (8.8)
+    //     group 4               3  7.4 -> 6.5 (8.2)   16 12.1 -> 8.9 (9.1)
+    //   head_dim 256, group 1   4 12.0 -> 8.2 (10.2)  16 28.0 -> 12.7 (11.1)
+    //     group 4               4 14.0 -> 8.2 (10.7)  16 28.1 -> 13.4 (11.8)
+    //   2 heads at least for group 1 up to 6 pages, head_dim 64 (3 pages, 2 KV heads,
+    //   2 -> 1: 5.9 -> 7.0)
+    // At head_dim 256 not where the workgroup is on its pages longer than the
+    // segments on theirs and a merge, which costs more for groups; with no partials to
+    // be had (a negative hint), or more than the allocation-free run has, the
+    // requests stay whole.
+    const int fewest = head_dim == 64 && group == 1 && max_pages <= 6 ? 2 : 1;
+    int few = hpw;
+    while (few > fewest && 2 * requests * heads <= slots * few) few /= 2;
     const int64_t longest = segs > 0 ? (total + segs - 1) / segs : 0;
-    const int64_t alone = head_dim == 256 ? 6 : group == 8 ? 8 : 16;  // pages of a head
-    if (head_dim != 128 && max_pages > 1 && max_pages <= kSmallMaxPages &&
-        (num_segments_hint < 0 || (max_pages - 2 * longest) * hpw <= alone ||
-         partials(cut) > KVC_NOALLOC_SCRATCH_BYTES) &&
-        (4 * requests * heads >= 3 * waves ||
-         requests * heads <= (group == 1 ? 1 : 2) * slots * hpw || !fits)) {
+    const int64_t alone = group == 1 ? 6 : group == 2 ? 10 : 14;  // pages of a head
+    const bool whole =
+        max_pages > 1 && max_pages <= kSmallMaxPages &&
+        (head_dim == 128 ? !lds
+                         : (4 * requests * heads >= 3 * waves ||
+                            requests * heads <= (group == 1 ? 1 : 2) * slots * hpw || !fits) &&
+                               (head_dim == 64 || num_segments_hint < 0 ||
+                                (max_pages - 2 * longest) * few <= alone ||
+                                partials(cut) > KVC_NOALLOC_SCRATCH_BYTES));
+    if (whole) {
+      hpw = few;
       cut.clear();
       for (int i = 0; i < batch; ++i)
         if (indptr_host[i + 1] > indptr_host[i]) cut.push_back(indptr_host[i]);
