@@ -991,10 +991,12 @@ __global__ __launch_bounds__((64 * (kNarrow ? kMaxWaveHeads : WaveCfg<G, D>::kWa
 
   // This wave's units of PU consecutive pages: unit ts, ts + TS, ... of the
   // segment; the pages' ids one per lane (a wave that shares the segment has at most
-  // half of its pages).
+  // half of its pages; at head_dim 64 the second register stays all the same, for the
+  // code that the compiler makes of it: 8 KV heads, group 8, 16 requests of 8000
+  // 56.8 us without, 55.4 with; of one request of 96 tokens, 2 heads 9.0 and 8.6).
   const int nw = n > PU * ts ? (n - PU * ts + PU * TS - 1) / (PU * TS) : 0;
   auto page_slot = [&](int j, int x) { return g0 + PU * (ts + TS * j) + x; };
-  constexpr int IR = kNarrow ? kIdRegs : kIdRegs / 2;
+  constexpr int IR = kNarrow || D == 64 ? kIdRegs : kIdRegs / 2;
   static_assert(kNarrow || W >= 2 * kMaxWaveHeads, "two waves at least share a segment");
   int32_t idr[IR];
   {
