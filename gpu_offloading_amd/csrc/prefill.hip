@@ -835,15 +835,22 @@ int64_t plan_ints_for(int64_t items, int hkv) {
 // took 90 us: up to a piece's length is lost at the end, and 400 partials of
 // 131 KB are written and read where this leaves 300.)
 // A unit or piece costs its key tiles + kUnitCost (its start and end, 4.6-6.4 us
-// against 1.6 us per tile) and the second launch kMergeCost; units stay whole
-// unless cutting them is a tenth sooner by that.  Units of up to kSplitTiles
-// tiles are never cut (with units of 11 on cut, a prefill of 1100 tokens took
-// 37.8 us against 33.7), and batches of more than kSplitMaxUnits units fill the
-// chip as they are.
+// against 1.6 us per tile) and the second launch kMergeCost, with a tile more for
+// every kPartsPerTile full partials above kFreeParts (of 131 KB: half the L2s);
+// units stay whole unless cutting them is a tenth sooner by that.  Whole and split,
+// us (chunks of queries over cached tokens): 3 of 300-600 over 1500-3000, 8 KV heads,
+// group 4 (391 partials; whole now) 76 and 93; 5 of 750-1500 over as many, group 1
+// (352, whole) 69 and 82; 8 of 100-200 over 750-1500, 4 heads, group 1 (140, split)
+// 43 and 36; 8 of 300-600 over 3000-6000, 8 heads, group 1 (368, split) 139 and 115.
+// Units of up to kSplitTiles tiles are never cut (with units of 11 on cut, a prefill
+// of 1100 tokens took 37.8 us against 33.7), and batches of more than kSplitMaxUnits
+// units fill the chip as they are.
 constexpr int kSplitTiles = 16;
 constexpr int kMinPiece = 4;       // tiles; shorter ones are mostly start and end
 constexpr int kUnitCost = 4;
 constexpr int kMergeCost = 5;       // the merge launch, in tiles
+constexpr int64_t kFreeParts = 128;
+constexpr int64_t kPartsPerTile = 16;
 constexpr int64_t kSplitMaxUnits = 512;
 
 // End of the longest workgroup when units of these costs are dealt longest
@@ -873,10 +880,13 @@ struct Piece {
 // little more where the rest of a unit would be shorter than kMinPiece).
 // Consecutive workgroups get consecutive tiles, head by head: the query tiles of
 // one request and head are near each other.  Returns the largest cost, or -1 if
-// kMaxWorkgroups are too few.
+// kMaxWorkgroups are too few; *parts counts the query tokens of the cut units'
+// pieces.
 int64_t deal(const std::vector<int32_t>& rec, int64_t n, int hkv, int64_t share,
-             std::vector<std::vector<Piece>>* lists) {
+             std::vector<std::vector<Piece>>* lists, int64_t* parts = nullptr,
+             int tile_tokens = 1) {
   int64_t w = 0, load = 0, most = 0;
+  if (parts) *parts = 0;
   if (lists) lists->assign(1, {});
   auto next = [&]() {
     ++w;
@@ -900,13 +910,16 @@ int64_t deal(const std::vector<int32_t>& rec, int64_t n, int hkv, int64_t share,
         first += take;
         ++index;
       } while (left > 0);
+      if (parts && index > 1)
+        *parts += index * std::min(tile_tokens,
+                                   rec[i * kItemInts + 2] - rec[i * kItemInts + 1]);
     }
   return most;
 }
 
 // The workgroups' share that ends a batch of these units soonest, or 0 to leave
 // them whole (unless splitting saves a tenth).
-int64_t split_share(const std::vector<int32_t>& rec, int64_t n, int hkv) {
+int64_t split_share(const std::vector<int32_t>& rec, int64_t n, int hkv, int tile_tokens) {
   if (n * hkv > kSplitMaxUnits) return 0;
   int64_t total = 0;
   int longest = 0;
@@ -926,8 +939,11 @@ int64_t split_share(const std::vector<int32_t>& rec, int64_t n, int hkv) {
     if (deal(rec, n, hkv, mid, nullptr) >= 0) hi = mid;
     else lo = mid + 1;
   }
-  const int64_t most = deal(rec, n, hkv, lo, nullptr);
-  return most >= 0 && most + kMergeCost < whole - whole / 10 ? lo : 0;
+  int64_t parts = 0;
+  const int64_t most = deal(rec, n, hkv, lo, nullptr, &parts, tile_tokens);
+  const int64_t merge =
+      kMergeCost + std::max<int64_t>(0, parts / tile_tokens - kFreeParts) / kPartsPerTile;
+  return most >= 0 && most + merge < whole - whole / 10 ? lo : 0;
 }
 
 // int32 entries of a split plan's image: the workgroups' table, the unit
@@ -1115,7 +1131,7 @@ int prefill_plan(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host,
     *split = kvc_prefill_split{};
     split->num_workgroups = int32_t(plan_workgroups(n, num_kv_heads));
     split->num_units = int32_t(n * num_kv_heads);
-    const int64_t share = split_share(rec, n, num_kv_heads);
+    const int64_t share = split_share(rec, n, num_kv_heads, tile_tokens);
     if (share > 0)
       return split_plan(rec, n, num_kv_heads, share, tile_tokens, group, sched, split, plan_host,
                         plan_capacity);

@@ -101,6 +101,18 @@ def test_split_plan_covers_every_key_once(q_lens, kv_lens, group, hkv, causal, c
     assert not by_unit and len(folded) == split.num_merges
 
 
+@pytest.mark.parametrize("q_lens,cached,group,hkv,cut", [
+    ([388, 510, 537], [2338, 2326, 1937], 4, 8, False),             # 391 full partials
+    ([1191, 1257, 1163, 1149, 1424], [1291, 1129, 859, 1104, 1101], 1, 8, False),   # 352
+    ([115, 152, 130, 138, 145, 166, 123, 194], [994, 1397, 1137, 1121, 833, 860, 1180, 1426], 1, 4, True),
+    ([374, 392], [6335, 8879], 8, 8, True),                         # long enough for many
+    ([1] * 40, [3000] * 40, 8, 4, True)])                           # partials of 8 rows
+def test_many_partials_over_short_units_stay_whole(q_lens, cached, group, hkv, cut):
+    kv_lens = [q + c for q, c in zip(q_lens, cached)]
+    split = _plan(q_lens, kv_lens, group, hkv, 1)[2]
+    assert (split.num_parts > 0) == cut, split.num_parts
+
+
 def _check(gpu, q_lens, kv_lens, group, hkv, seed, causal, hide=()):
     q, kc, vc, qo, kvi, idx, lpl = _case(q_lens, kv_lens, group * hkv, hkv, seed, device=gpu)
     idx = idx.copy()
