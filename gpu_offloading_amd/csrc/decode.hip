@@ -1962,7 +1962,10 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
   // Many requests per segment of the wave kernel: its waves would share every
   // request and meet at its end.  The narrow form, a wave per head and segment,
   // closes pieces without meeting; its segments are as many as the chip has waves
-  // for (at most 8 per CU, at least two pages each), or three quarters of that.  It
+  // for (at most 8 per CU, at least two pages each), or three quarters of that (seven
+  // eighths for groups 2 and 4 at head_dim 64: five sixths of them take 54.7 us
+  // against the other form's 52.7 for 20 of 1100-11000 tokens, 8 KV heads, 35.9
+  // against 33.2 for 40 of 2000-5000, 4 heads; group 8 53.3 against 54.0).  It
   // is taken where a request has at most about kSpecParts of them, so that the
   // merge stays one batch of loads, where they are more than the other form runs at
   // once, and where its partials fit the allocation-free run or are no more than
@@ -1981,7 +1984,8 @@ extern "C" int kvc_decode_plan(const int32_t* indptr_host, const int32_t* last_p
     int64_t narrow =
         std::min({std::max<int64_t>(1, waves / heads), total / 2, kNarrowPerCu * slots});
     const int64_t most = kSpecParts * requests;
-    if (4 * most * heads >= 3 * waves) narrow = std::min(narrow, most);
+    const int eighths = head_dim == 64 && (group == 2 || group == 4) ? 7 : 6;
+    if (8 * most * heads >= eighths * waves) narrow = std::min(narrow, most);
     const bool fits = num_segments_hint == 0 && head_dim < 256 && narrow <= most &&
                       2 * narrow * heads > 3 * slots * hpw;
     auto partials = [&](const std::vector<int64_t>& c) {

@@ -89,3 +89,11 @@ def test_random_plans_of_every_layout(lib, seed):  # noqa: F811
         assert sched.num_head_groups * sched.heads_per_group == hkv
         few = _plan(lib, lens, hq=hkv * group, hkv=hkv, d=d, cus=cus, hint=-1)[1]
         assert sched.workspace_bytes <= max(16 << 20, few.workspace_bytes)
+
+
+def test_narrow_segments_leave_few_waves_out(lib):  # noqa: F811
+    # 20 requests, at most 16 segments each: 320 of the 384 that the chip has waves for
+    lens = [1100 + 500 * i for i in range(20)]
+    for group, want in ((2, 128), (4, 128), (8, 320)):
+        assert _plan(lib, lens, hq=8 * group, hkv=8, d=64)[1].num_segments == want
+    assert _plan(lib, lens * 2, hq=32, hkv=8, d=64)[1].num_segments == 384
